@@ -54,6 +54,8 @@ SIGNATURES = {
     "parcae_step": (_int, [_vp, _vp, _vp, _vp, _vp, _f32, _vp, _vp, _vp, _int, _int, _int, _vp]),
     "distogram_expected_distance": (_int, [_vp, _vp, _vp, _vp, _vp, _int, _int, _int, _int, _vp]),
     "abs_diff_quantile": (_int, [_vp, _vp, _sz, _f32, _vp, _vp]),
+    "abs_diff_quantile_workspace_bytes": (_sz, [_sz]),
+    "abs_diff_quantile_ws": (_int, [_vp, _vp, _sz, _f32, _vp, _vp, _sz, _vp]),
     "q8_linear": (_int, [_vp, _vp, _vp, _vp, _vp, _int, _int, _int, _int, _vp]),
     "q8_linear_ws": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _int, _int, _int, _int, _vp, _sz, _vp]),
     "q8_linear_noalloc": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _int, _int, _int, _int, _vp]),

@@ -848,11 +848,29 @@ int distogram_expected_distance(const float* r, const esm_half* w, const float* 
   return hip_status(esm::launch_expected_distance(args, grid, (hipStream_t)stream), "distogram_expected_distance launch");
 }
 
+size_t abs_diff_quantile_workspace_bytes(size_t n) { return esm::abs_diff_quantile_ws_size(n); }
+
+static int quantile_impl(const char* fn, const float* x, const float* y, size_t n, float q, float* out, void* ws,
+                         void* stream) {
+  if (n == 0) return fail(ESM_ERR_SHAPE, "%s: n must be >= 1", fn);
+  if (!(q >= 0.f && q <= 1.f)) return fail(ESM_ERR_SHAPE, "%s: q=%g outside [0, 1]", fn, (double)q);
+  if (!x || !out) return fail(ESM_ERR_NULL, "%s: NULL pointer", fn);
+  return hip_status(esm::launch_abs_diff_quantile(x, y, n, q, out, ws, (hipStream_t)stream), "abs_diff_quantile launch");
+}
+
 int abs_diff_quantile(const float* x, const float* y, size_t n, float q, float* out, void* stream) {
-  if (n == 0) return fail(ESM_ERR_SHAPE, "abs_diff_quantile: n must be >= 1");
-  if (!(q >= 0.f && q <= 1.f)) return fail(ESM_ERR_SHAPE, "abs_diff_quantile: q=%g outside [0, 1]", (double)q);
-  if (!x || !out) return fail(ESM_ERR_NULL, "abs_diff_quantile: NULL pointer");
-  return hip_status(esm::launch_abs_diff_quantile(x, y, n, q, out, (hipStream_t)stream), "abs_diff_quantile launch");
+  return quantile_impl("abs_diff_quantile", x, y, n, q, out, nullptr, stream);
+}
+
+int abs_diff_quantile_ws(const float* x, const float* y, size_t n, float q, float* out, void* workspace,
+                         size_t workspace_bytes, void* stream) {
+  const size_t need = esm::abs_diff_quantile_ws_size(n);
+  if (workspace) {
+    if (workspace_bytes < need)
+      return fail(ESM_ERR_SHAPE, "abs_diff_quantile_ws: workspace of %zu bytes, needs %zu", workspace_bytes, need);
+    if (!aligned16(workspace)) return fail(ESM_ERR_ALIGN, "abs_diff_quantile_ws: workspace must be 16-byte aligned");
+  }
+  return quantile_impl("abs_diff_quantile_ws", x, y, n, q, out, workspace, stream);
 }
 
 size_t q8_packed_scales_bytes(int N, int K) {

@@ -212,7 +212,10 @@ hipError_t launch_transition(const TransitionArgs& a, int grid, hipStream_t s);
 hipError_t launch_esmc_ln(const EsmcLnArgs& a, hipStream_t s);
 hipError_t launch_parcae_step(const ParcaeArgs& a, int grid, hipStream_t s);
 hipError_t launch_expected_distance(const DistoArgs& a, int grid, hipStream_t s);
-hipError_t launch_abs_diff_quantile(const float* x, const float* y, size_t n, float q, float* out, hipStream_t s);
+// ws: abs_diff_quantile_ws_size(n) bytes (0: none needed), or nullptr (one workgroup whatever n).
+size_t abs_diff_quantile_ws_size(size_t n);
+hipError_t launch_abs_diff_quantile(const float* x, const float* y, size_t n, float q, float* out, void* ws,
+                                    hipStream_t s);
 hipError_t launch_esmc_qk_rope(const EsmcRopeArgs& a, hipStream_t s);
 hipError_t launch_esmc_attention(const EsmcAttnArgs& a, hipStream_t s);
 hipError_t launch_esmc_swiglu(const half_t* x12, half_t* y, size_t M, int F, hipStream_t s);

@@ -257,8 +257,8 @@ __global__ __launch_bounds__(256, 1) void expected_distance_kernel(DistoArgs p) 
 }
 
 // ---- quantile of |x - y| ----------------------------------------------------------------------
-// Beyond the register-held sizes (abs_diff_quantile_regs_kernel below): one workgroup of QT
-// threads. Radix selection on the bit patterns of the non-negative values (their order is the
+// Beyond the register-held sizes (abs_diff_quantile_regs_kernel below) for a caller without a
+// workspace: one workgroup of QT threads. Radix selection on the bit patterns of the non-negative values (their order is the
 // value order): 3 passes of 11, 11 and 10 bits, each a histogram of the candidates still
 // matching the selected high bits, for the two ranks that bracket the quantile at once; then
 // linear interpolation between the two order statistics (the definition of torch.quantile).
@@ -580,6 +580,165 @@ __global__ __launch_bounds__(QR) void abs_diff_quantile_regs_kernel(const float*
   }
 }
 
+// ---- the quantile over many workgroups --------------------------------------------------------
+// For the sizes the register-held kernel does not take, when the caller gives a workspace. One
+// workgroup streaming x and y three times is bound by what a single CU can read (103 us at 262,144
+// values, ~60 GB/s per pass); here every pass is spread over the chip and the kernel boundary
+// orders the histograms between passes: a clearing launch, three counting launches (11, 10 and
+// 10 bits under the zero sign bit) and a final selection, each a few microseconds long.
+// Back to back, one workgroup against this: 57,345 values 33 / 21 us, 262,144 (L = 512) 106 / 23,
+// 1,048,576 426 / 25, all values equal at 262,144 667 / 22; the register-held kernel below 57,345
+// values takes 18, so the line between the two stays where its registers end.
+// A counting workgroup first finds the bins of both ranks in the previous pass's histogram
+// (every workgroup repeats that scan of at most 2 x 2048 counters, which costs less than a launch
+// of its own), counts its values that match them in LDS, in 4 copies picked by the lane so that
+// equal neighbours do not queue on one counter, and adds its non-zero counters to the global
+// histogram. Same order statistics, so the same bits as the one-workgroup kernels.
+constexpr int SQT = 512, SQU = 8, SQB0 = 2048, SQB = 1024;
+constexpr int kSqShift[3] = {20, 10, 0};
+struct SpreadSel {            // after pass p: the selected high bits and the ranks below them
+  uint32_t prefix[2], pad[2];
+  unsigned long long rank[2];
+};
+struct SpreadWs {
+  uint32_t h0[SQB0];          // pass 0 (both ranks)
+  uint32_t h[2][2][SQB];      // passes 1, 2: per rank; one histogram while the ranks share their bits
+  SpreadSel sel[2];           // after passes 0 and 1
+};
+constexpr int kSpreadClear = SQB0 + 4 * SQB;  // words of histograms
+
+__global__ __launch_bounds__(SQT) void quantile_clear_kernel(SpreadWs* ws) {
+  const int i = blockIdx.x * SQT + threadIdx.x;
+  if (i < kSpreadClear) ws->h0[i] = 0u;  // h0 and h are contiguous
+}
+
+// Both ranks' state after pass P from the state before it and P's histogram(s): a workgroup-wide
+// exclusive scan of the counters, thread t owning NB / SQT consecutive ones.
+template <int P>
+DEV void spread_select(const SpreadWs* ws, size_t n, float q, SpreadSel& out, unsigned long long* rank_s, uint32_t* sel_s,
+                       uint32_t (*wsum)[SQT / 64]) {
+  constexpr int NB = P == 0 ? SQB0 : SQB, BPT = NB / SQT, NWV = SQT / 64;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  SpreadSel s;
+  if constexpr (P == 0) {
+    const double pos = (double)q * (double)(n - 1);
+    s.prefix[0] = s.prefix[1] = 0u;
+    s.rank[0] = (unsigned long long)pos;
+    s.rank[1] = s.rank[0] + 1 < n ? s.rank[0] + 1 : s.rank[0];
+  } else {
+    s = ws->sel[P - 1];
+  }
+  const bool shared = s.prefix[0] == s.prefix[1];
+  uint32_t cb[2][BPT], c[2], inc[2];
+#pragma unroll
+  for (int t = 0; t < 2; t++) {
+    const uint32_t* ht = P == 0 ? ws->h0 : ws->h[P == 0 ? 0 : P - 1][shared ? 0 : t];
+    c[t] = 0;
+#pragma unroll
+    for (int k = 0; k < BPT; k++) {
+      cb[t][k] = ht[BPT * tid + k];
+      c[t] += cb[t][k];
+    }
+    inc[t] = c[t];
+  }
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1)
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      const uint32_t o = __shfl_up(inc[t], off);
+      if (lane >= off) inc[t] += o;
+    }
+  if (lane == 63) {
+    wsum[0][wv] = inc[0];
+    wsum[1][wv] = inc[1];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < 2; t++) {
+    unsigned long long before = inc[t] - c[t];
+#pragma unroll
+    for (int w = 0; w < NWV; w++) before += w < wv ? wsum[t][w] : 0u;
+    if (s.rank[t] >= before && s.rank[t] < before + c[t]) {  // exactly one thread per rank
+      int k = 0;
+      while (k < BPT - 1 && s.rank[t] >= before + cb[t][k]) before += cb[t][k++];
+      sel_s[t] = (uint32_t)(BPT * tid + k);
+      rank_s[t] = s.rank[t] - before;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < 2; t++) {
+    out.prefix[t] = s.prefix[t] | (sel_s[t] << kSqShift[P]);
+    out.pad[t] = 0u;
+    out.rank[t] = rank_s[t];
+  }
+}
+
+template <int P>
+__global__ __launch_bounds__(SQT) void quantile_count_kernel(const float* __restrict__ x, const float* __restrict__ y,
+                                                             size_t n, float q, SpreadWs* ws) {
+  constexpr int NB = P == 0 ? SQB0 : SQB, NH = P == 0 ? 1 : 2, CP = 4;
+  constexpr uint32_t kNone = 0xffffffffu;
+  constexpr uint32_t mask = P == 0 ? 0u : ~((1u << kSqShift[P == 0 ? 0 : P - 1]) - 1u);  // bits already selected
+  __shared__ uint32_t hist[NH][NB * CP];
+  __shared__ unsigned long long rank_s[2];
+  __shared__ uint32_t sel_s[2], wsum[2][SQT / 64];
+  const int tid = threadIdx.x;
+  for (int k = tid; k < NH * NB * CP; k += SQT) (&hist[0][0])[k] = 0u;
+  SpreadSel s{};
+  if constexpr (P > 0) {
+    spread_select<P == 0 ? 0 : P - 1>(ws, n, q, s, rank_s, sel_s, wsum);
+    if (blockIdx.x == 0 && tid == 0) ws->sel[P == 0 ? 0 : P - 1] = s;  // read by the next launch
+  }
+  __syncthreads();
+  const bool shared = s.prefix[0] == s.prefix[1];
+  for (size_t c0 = (size_t)blockIdx.x * (SQT * SQU); c0 < n; c0 += (size_t)gridDim.x * (SQT * SQU)) {
+    const size_t cnt = n - c0 < (size_t)SQT * SQU ? n - c0 : (size_t)SQT * SQU;
+    const rsrc_t rx = make_rsrc_n(x + c0, (uint32_t)(cnt * 4));
+    const rsrc_t ry = make_rsrc_n(y ? y + c0 : x, y ? (uint32_t)(cnt * 4) : 0u);
+    uint32_t xb[SQU], yb[SQU];
+#pragma unroll
+    for (int j = 0; j < SQU; j++) {
+      xb[j] = __builtin_amdgcn_raw_buffer_load_b32(rx, tid * 4, SQT * 4 * j, 0);
+      yb[j] = __builtin_amdgcn_raw_buffer_load_b32(ry, tid * 4, SQT * 4 * j, 0);
+    }
+#pragma unroll
+    for (int j = 0; j < SQU; j++) {
+      const uint32_t u = __float_as_uint(fabsf(__uint_as_float(xb[j]) - __uint_as_float(yb[j]))) |
+                         ((uint32_t)(tid + SQT * j) < cnt ? 0u : kNone);
+      const uint32_t bin = ((u >> kSqShift[P]) & (NB - 1)) * CP + (tid & (CP - 1));
+      if (u != kNone && (u & mask) == s.prefix[0]) atomicAdd(&hist[0][bin], 1u);
+      if constexpr (NH == 2)
+        if (!shared && u != kNone && (u & mask) == s.prefix[1]) atomicAdd(&hist[1][bin], 1u);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < NH; t++) {
+    if (t == 1 && shared) break;
+    uint32_t* g = P == 0 ? ws->h0 : ws->h[P == 0 ? 0 : P - 1][t];
+    for (int k = tid; k < NB; k += SQT) {
+      const uint4 v = *reinterpret_cast<const uint4*>(&hist[t][CP * k]);
+      const uint32_t sum = v.x + v.y + v.z + v.w;
+      if (sum) atomicAdd(&g[k], sum);
+    }
+  }
+}
+
+__global__ __launch_bounds__(SQT) void quantile_final_kernel(const SpreadWs* ws, size_t n, float q,
+                                                             float* __restrict__ out) {
+  __shared__ unsigned long long rank_s[2];
+  __shared__ uint32_t sel_s[2], wsum[2][SQT / 64];
+  SpreadSel s;
+  spread_select<2>(ws, n, q, s, rank_s, sel_s, wsum);
+  if (threadIdx.x == 0) {
+    const double pos = (double)q * (double)(n - 1);
+    const float frac = (float)(pos - (double)(unsigned long long)pos);
+    const float a = __uint_as_float(s.prefix[0]), b = __uint_as_float(s.prefix[1]);
+    out[0] = a + frac * (b - a);
+  }
+}
+
 hipError_t launch_parcae_step(const ParcaeArgs& a, int grid, hipStream_t s) {
   if (a.C == 128)
     ESM_LAUNCH(parcae_step_kernel<128>, dim3(grid), dim3(256), 0, s, a);
@@ -604,11 +763,24 @@ hipError_t launch_expected_distance(const DistoArgs& a, int grid, hipStream_t s)
   return hipGetLastError();
 }
 
-hipError_t launch_abs_diff_quantile(const float* x, const float* y, size_t n, float q, float* out, hipStream_t s) {
-  if (n <= (size_t)QR * QCR)
+size_t abs_diff_quantile_ws_size(size_t n) { return n <= (size_t)QR * QCR ? 0 : sizeof(SpreadWs); }
+
+hipError_t launch_abs_diff_quantile(const float* x, const float* y, size_t n, float q, float* out, void* ws,
+                                    hipStream_t s) {
+  if (n <= (size_t)QR * QCR) {
     ESM_LAUNCH(abs_diff_quantile_regs_kernel, dim3(1), dim3(QR), 0, s, x, y, (uint32_t)n, q, out);
-  else
+  } else if (ws) {
+    SpreadWs* w = static_cast<SpreadWs*>(ws);
+    const size_t chunks = (n + SQT * SQU - 1) / (SQT * SQU);
+    const dim3 grid((unsigned)(chunks < 1024 ? chunks : 1024));
+    ESM_LAUNCH(quantile_clear_kernel, dim3((kSpreadClear + SQT - 1) / SQT), dim3(SQT), 0, s, w);
+    ESM_LAUNCH((quantile_count_kernel<0>), grid, dim3(SQT), 0, s, x, y, n, q, w);
+    ESM_LAUNCH((quantile_count_kernel<1>), grid, dim3(SQT), 0, s, x, y, n, q, w);
+    ESM_LAUNCH((quantile_count_kernel<2>), grid, dim3(SQT), 0, s, x, y, n, q, w);
+    ESM_LAUNCH(quantile_final_kernel, dim3(1), dim3(SQT), 0, s, w, n, q, out);
+  } else {
     ESM_LAUNCH(abs_diff_quantile_kernel, dim3(1), dim3(QT), 0, s, x, y, n, q, out);
+  }
   return hipGetLastError();
 }
 

@@ -241,7 +241,11 @@ def abs_diff_quantile(x, y=None, q: float = 0.95, out=None):
         if y.numel() != x.numel():
             raise capi.EsmError(-2, "abs_diff_quantile: x and y differ in size")
     out = torch.empty(1, dtype=torch.float32, device=x.device) if out is None else _out(out, "out", torch.float32, 1)
-    capi.check(lib.abs_diff_quantile(x.data_ptr(), _ptr(y), x.numel(), float(q), out.data_ptr(), capi.stream_ptr()))
+    n = x.numel()
+    need = int(lib.abs_diff_quantile_workspace_bytes(n))
+    ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None  # many workgroups from 57,345 values
+    capi.check(lib.abs_diff_quantile_ws(x.data_ptr(), _ptr(y), n, float(q), out.data_ptr(), _ptr(ws), need,
+                                        capi.stream_ptr()))
     return out
 
 

@@ -427,12 +427,19 @@ int esmc_swiglu(const esm_half* x12, esm_half* y, int M, int F, void* stream);
  *   Exact (order statistics by radix selection). x, y [n] fp32; out one fp32. A NaN difference
  *   orders above +inf, as the sort of the MLX loop's p95 (var_6b_mlx_loop.py:78-84) orders it
  *   (torch.quantile would return NaN instead).
+ * abs_diff_quantile_ws: the same value with a workspace of
+ *   abs_diff_quantile_workspace_bytes(n) bytes (16-byte aligned; 0: not used), which lets
+ *   large n run on many workgroups. workspace NULL: as abs_diff_quantile; below the size:
+ *   ESM_ERR_SHAPE.
  */
 int parcae_step(const float* z, const float* z_init, const float* refined, const float* ln_w, const float* ln_b,
                 float eps, const float* a, const esm_half* b_mat, float* z_out, int B, int L, int C, void* stream);
 int distogram_expected_distance(const float* r, const esm_half* w, const float* bias, const float* centers, float* ed,
                                 int B, int L, int C, int nbins, void* stream);
 int abs_diff_quantile(const float* x, const float* y, size_t n, float q, float* out, void* stream);
+size_t abs_diff_quantile_workspace_bytes(size_t n);
+int abs_diff_quantile_ws(const float* x, const float* y, size_t n, float q, float* out, void* workspace,
+                         size_t workspace_bytes, void* stream);
 
 /*
  * q8_linear_ws without a workspace, for callers that cannot allocate device memory (code

@@ -118,6 +118,33 @@ def test_abs_diff_quantile_one_value(gpu_lib, pkg, n):
     assert got == float(torch.quantile(x.double(), 0.95))
 
 
+@pytest.mark.parametrize("n", [57345, 61440, 61441, 600001])
+@pytest.mark.parametrize("kind", ["random", "one value", "two bins", "infinities and NaN"])
+def test_abs_diff_quantile_many_workgroups(gpu_lib, pkg, n, kind):
+    """The many-workgroup form (a workspace, past the register-held sizes) returns the bits of the
+    one-workgroup form: at its smallest size, one whole chunk of 4,096 values more or less, and
+    beyond; an undersized workspace is refused."""
+    lib, g = pkg.capi.lib(), torch.Generator().manual_seed(n)
+    x, y = torch.randn(n, generator=g) * 3, torch.randn(n, generator=g)
+    if kind == "one value":
+        x, y = torch.full((n,), 2.5), torch.zeros(n)
+    elif kind == "two bins":
+        x, y = torch.where(torch.rand(n, generator=g) < 0.5, 1.25, 768.0), torch.zeros(n)
+    elif kind == "infinities and NaN":
+        x[::7], x[3::41], y[5::1000] = float("inf"), float("nan"), 0.0
+    x, y = x.to(DEV), y.to(DEV)
+    need = lib.abs_diff_quantile_workspace_bytes(n)
+    ws = torch.full((need,), 255, dtype=torch.uint8, device=DEV)  # the call clears what it uses
+    a, b = torch.empty(1, device=DEV), torch.empty(1, device=DEV)
+    st = pkg.capi.stream_ptr()
+    for q in (0.0, 0.5, 0.8571, 0.95, 1.0):
+        pkg.capi.check(lib.abs_diff_quantile(x.data_ptr(), y.data_ptr(), n, q, a.data_ptr(), st))
+        pkg.capi.check(lib.abs_diff_quantile_ws(x.data_ptr(), y.data_ptr(), n, q, b.data_ptr(), ws.data_ptr(), need, st))
+        assert torch.equal(a.view(torch.int32), b.view(torch.int32)), q
+    assert lib.abs_diff_quantile_workspace_bytes(57344) == 0
+    assert lib.abs_diff_quantile_ws(x.data_ptr(), None, n, 0.5, b.data_ptr(), ws.data_ptr(), need - 1, st) == -2
+
+
 def _oracle_trunk(blocks):
     f = ("w_bundle", "w_emit", "w_gate", "ln_in_w", "ln_in_b", "ln_mix_w", "ln_mix_b", "ln_in_eps", "ln_mix_eps",
          "outgoing")
