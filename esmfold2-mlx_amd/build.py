@@ -22,7 +22,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB_NAME = "libesmfold2_amd.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
 SOURCES = ["project.hip", "contract.hip", "epilogue.hip", "q8.hip", "transition.hip", "esmc.hip",
-           "recycle.hip", "wide.hip", "capi.cpp"]
+           "recycle.hip", "wide.hip", "stream.hip", "capi.cpp"]
 HEADERS = ["common.h", "kernels.h", os.path.join("..", "..", "include", "esmfold2_amd.h")]
 ARCH = "gfx950"
 

@@ -665,6 +665,15 @@ static bool narrow_transition(int C, int H, bool swiglu) {
   return C == 128 && (swiglu ? H == 256 : (H == 256 || H == 512));
 }
 
+// At C = 256 the whole transition is one cell-stationary kernel when its tiles of 256 cells reach more
+// than a quarter of the CUs. Below that the split into three launches, which spreads a small grid over
+// more CUs, is shorter (us, three launches against one, SwiGLU H = 1024 on 256 CUs: L = 76 53 / 70, L =
+// 100 60 / 72, L = 128 (64 tiles) 68 / 75, L = 160 120 / 79, L = 238 174 / 108; ReLU L = 128 59 / 54). At
+// C = 128 the register-resident kernel is the shorter one at most sizes (L = 238 26 / 24, L = 476 81 / 98).
+static bool stream_transition(int C, int H, size_t ncells) {
+  return C == 256 && (size_t)H * C <= (1u << 29) && 4 * ((ncells + 255) / 256) > (size_t)cu_count();
+}
+
 size_t pair_transition_workspace_bytes(int B, int L, int C, int hidden, int swiglu) {
   if (B <= 0 || L <= 0 || C <= 0 || hidden <= 0 || narrow_transition(C, hidden, swiglu != 0)) return 0;
   const size_t cells = (size_t)B * L * L;
@@ -702,6 +711,10 @@ int pair_transition_ws(const esm_half* z, esm_half* out, const float* ln_w, cons
     return fail(ESM_ERR_SHAPE, "pair_transition: workspace of %zu bytes, %zu needed", workspace_bytes, need);
   if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0)
     return fail(ESM_ERR_ALIGN, "pair_transition: workspace must be 256-byte aligned");
+  if (stream_transition(C, hidden, ncells)) {
+    esm::TransitionArgs a{H(z), H(out), ln_w, ln_b, eps, H(w1), w2 ? H(w2) : nullptr, H(w3), ncells, 0, hidden};
+    return hip_status(esm::launch_transition_stream(a, C, cu_count(), st), "pair_transition launch");
+  }
   half_t* wn = static_cast<half_t*>(workspace);
   half_t* wh = wn + (ncells * C * sizeof(esm_half) + 255) / 256 * 256 / sizeof(esm_half);
   hipError_t e = esm::launch_ln_rows(z, nullptr, false, ln_w, ln_b, eps, wn, ncells, C, st);

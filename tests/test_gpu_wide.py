@@ -178,6 +178,31 @@ def test_transition_256_h1024_across_line_tiles(gpu_lib, pkg, L, swiglu):
     _bar(out, ref, z)
 
 
+@pytest.mark.parametrize("B,L,H", [(1, 129, 32), (2, 91, 64), (1, 129, 96), (1, 128, 128), (1, 181, 160),
+                                   (1, 257, 128)])
+@pytest.mark.parametrize("swiglu", [True, False])
+def test_transition_256_one_launch(gpu_lib, pkg, B, L, H, swiglu):
+    # the cell-stationary kernel (more than 64 tiles of 256 cells on 256 CUs; L = 128 is the last of
+    # the three-launch form): one to five steps of its weight ring, waves with some or no cells in
+    # the last tile, one and two rounds of tiles; in place
+    C = 256
+    g = torch.Generator().manual_seed(L + H + swiglu)
+    z = (0.5 + torch.randn(B, L, L, C, generator=g)).half()  # (outputs below 16: half an fp16 ulp stays under the bar)
+    w1 = torch.randn(H, C, generator=g) * C ** -0.5
+    w2 = torch.randn(H, C, generator=g) * C ** -0.5 if swiglu else None
+    w3 = torch.randn(C, H, generator=g) * H ** -0.5
+    lw, lb = 1 + 0.3 * torch.randn(C, generator=g), 0.3 * torch.randn(C, generator=g)
+    tr = pkg.trunk.PairTransition(lw, lb, w1, w3, w2=w2)
+    zd = z.to(DEV)
+    out = tr(zd)
+    p = otr.TransitionWeights(lw, lb, w1.half().float(), w3.half().float(), None if w2 is None else w2.half().float())
+    with torch.no_grad():
+        ref = otr.transition(z.float(), p)
+    _bar(out, ref, z)
+    tr.run(zd, zd)
+    assert torch.equal(zd, out)
+
+
 @pytest.mark.parametrize("C,L", [(384, 129), (384, 257), (512, 65), (512, 129)])
 @pytest.mark.parametrize("outgoing", [True, False])
 def test_tmu_384_512_across_tiles(gpu_lib, pkg, C, L, outgoing):
