@@ -288,6 +288,14 @@ int tmu_epilogue(const esm_half* x, int ldx, const esm_half* z, const esm_half* 
   return hip_status(esm::launch_epilogue(e, grid, (hipStream_t)stream), "tmu_epilogue launch");
 }
 
+// At C = 256 the update's emit / gate step is one cell-stationary kernel with both LayerNorms once its units
+// of 32 cells of a row outnumber half the CUs; below that one unit's latency exceeds the two launches it
+// replaces (whole update, us, two launches / one: L = 48 30.9 / 32.1, L = 64 (128 units) 34.2 / 34.9, L = 65
+// 39.8 / 37.2, L = 76 43.1 / 39.2, L = 128 53.8 / 48.4, L = 238 141 / 115, L = 476 554 / 462).
+static bool stream_emit(int C, int B, int L) {
+  return C == 256 && 2LL * B * L * ((L + 31) / 32) > cu_count();
+}
+
 // The wide path of tmu_forward (C = c, a multiple of 128 other than 128, up to 512): five
 // launches in the workspace planes a | b | x | n (x / 256 as in the narrow path):
 //   n = LN_in(z) (cell-major)  ->  a, b = gate(n W^T) (channel-major, GATE_CM)  ->  x = a b^T
@@ -339,6 +347,12 @@ static int tmu_forward_wide(const esm_half* z, const esm_half* mask, const float
   esm::ContractArgs ca{wa, wb, wx, B * c, L, ld, ld, kScale, frag ? 1 : 0};
   e = esm::launch_contract(ca, st);
   if (e != hipSuccess) return hip_status(e, "tmu_forward contract launch");
+  if (stream_emit(C, B, L)) {
+    esm::EpilogueArgs ea{wx, ld, H(z), mask ? H(mask) : nullptr, ln_in_w, ln_in_b, ln_in_eps, ln_mix_w, ln_mix_b,
+                         ln_mix_eps * kScale * kScale, H(w_emit), H(w_gate), H(out), B, L, residual ? 1 : 0,
+                         out_mask ? 1 : 0, 0, 0};
+    return hip_status(esm::launch_emit_stream(ea, st), "tmu_forward emit launch");
+  }
   e = esm::launch_ln_cf_to_cl(wx, ld, ln_mix_w, ln_mix_b, ln_mix_eps * kScale * kScale, wa, B, L, c, st);
   if (e != hipSuccess) return hip_status(e, "tmu_forward ln_cf_to_cl launch");
   esm::WideArgs r{};

@@ -10,21 +10,25 @@ namespace esm {
 namespace {
 constexpr int kCsWaves = 8;                  // two per SIMD: one's VALU work runs under the other's MFMAs
 constexpr int kCsThreads = 64 * kCsWaves;
+constexpr int kEmWaves = 4;                  // of the kernels that run two workgroups per CU
 constexpr int kCsCells = 32;                 // cells per wave: the columns of one 32x32x16 MFMA
 
 // 1 KB of a matrix into LDS, 16 bytes per lane from anywhere in the resource, landing in lane order
 // at a wave-uniform LDS address. Written as assembly because the compiler, which cannot tell a
 // ring's slots apart, waits for every such load in flight before the next LDS read; here the wait is
 // where the slot is handed over (wait_vm and a barrier). Nothing is written to a register.
+// (A uniform value computed in vector registers, an integer division's say, has to be moved to a scalar
+// one by hand for an assembly operand; the waits inside cover that move too.)
+DEV uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 typedef u32x4 dma_src_t;
 DEV dma_src_t dma_src(const void* base, uint32_t bytes) {
   const uint64_t a = reinterpret_cast<uint64_t>(base);
-  return u32x4{(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, bytes, (uint32_t)kBufWord3};
+  return u32x4{uniform((uint32_t)a), uniform((uint32_t)(a >> 32) & 0xffffu), uniform(bytes), (uint32_t)kBufWord3};
 }
 DEV void dma16(dma_src_t r, uint32_t l, uint32_t off, uint32_t soff) {
   __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                    :
-                   : "s"(l), "v"(off), "s"(r), "s"(soff)
+                   : "s"(uniform(l)), "v"(off), "s"(r), "s"(uniform(soff))
                    : "memory");
 }
 #define wait_vm(N) \
@@ -45,6 +49,68 @@ DEV float lane_sum(float v) {
 }
 // Ends a value's live range in other forms: the next use starts from these registers.
 DEV void pin(half8& v) { __asm__ volatile("" : "+v"(v)); }
+// The lane number, formed anew at each use: where the registers are full, addresses are computed from it
+// instead of being kept.
+DEV int fresh_lane() {
+  int l;
+  __asm__ volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+  return l;
+}
+// LayerNorm in place of a wave's 32 cells in LDS (rows of C halfs, 16-byte piece j of cell c at
+// j ^ (c % (C / 8))), two-pass fp32 statistics, 1 KB at a time in a rolled loop: straight-line code that
+// runs once per tile is bound by its instruction fetches (unrolled, staging and LayerNorm took 36 us
+// of a launch at one tile per CU instead of 20).
+template <int C>
+DEV void ln_rows_lds(char* zs, const float* w, const float* b, float eps) {
+  constexpr int LPC = C / 8, CPI = 64 / LPC;  // lanes per cell, cells per KB
+  const int l = fresh_lane(), l0 = l & (LPC - 1), cl = l / LPC;
+  float g[8], bb[8];
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    g[e] = w[8 * l0 + e];
+    bb[e] = b[8 * l0 + e];
+  }
+#pragma unroll 4
+  for (int i = 0; i < kCsCells / CPI; i++) {
+    char* piece = zs + i * 1024 + cl * (2 * C) + 16 * (l0 ^ ((i * CPI + cl) & (LPC - 1)));
+    const half8 x = *reinterpret_cast<const half8*>(piece);
+    const half2v one = {(half_t)1.0f, (half_t)1.0f};
+    const float s0 = __builtin_amdgcn_fdot2(half2v{x[2], x[3]}, one,
+                                            __builtin_amdgcn_fdot2(half2v{x[0], x[1]}, one, 0.f, false), false);
+    const float s1 = __builtin_amdgcn_fdot2(half2v{x[6], x[7]}, one,
+                                            __builtin_amdgcn_fdot2(half2v{x[4], x[5]}, one, 0.f, false), false);
+    const float mean = lane_sum<LPC>(s0 + s1) * (1.0f / C);
+    float q0 = 0.f, q1 = 0.f, d[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) d[e] = (float)x[e] - mean;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      q0 += d[e] * d[e];
+      q1 += d[e + 4] * d[e + 4];
+    }
+    const float rstd = rsqrtf(lane_sum<LPC>(q0 + q1) * (1.0f / C) + eps);
+    half8 v;
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] = (half_t)(d[e] * rstd * g[e] + bb[e]);
+    *reinterpret_cast<half8*>(piece) = v;
+  }
+}
+// The rows' MFMA fragments: channels 16 k + 8 (lane / 32) .. + 7 of cell lane % 32.
+template <int C>
+DEV void rows_to_frags(const char* zs, half8 (&f)[C / 16]) {
+  const int l = fresh_lane();
+#pragma unroll
+  for (int k = 0; k < C / 16; k++)
+    f[k] = *reinterpret_cast<const half8*>(zs + (l & 31) * (2 * C) + 16 * ((2 * k + (l >> 5)) ^ (l & (C / 8 - 1))));
+#pragma unroll
+  for (int k = 0; k < C / 16; k++) pin(f[k]);
+}
+// The rows' accumulator pieces: channels 4 j2 + 0..3 with j2 = 2 (4 ob + q) + lane / 32, as the 32x32
+// MFMA leaves rows 8 q + 4 (lane / 32) + 0..3 of output block ob for cell lane % 32.
+template <int C>
+DEV char* acc_piece(char* zs, int l, int ob, int q) {
+  return zs + (l & 31) * (2 * C) + 8 * (l >> 5) + 16 * ((4 * ob + q) ^ (l & (C / 8 - 1)));
+}
 DEV void cs_lds_fence() {  // a wave's own LDS operations complete in order: a compiler fence only
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -83,7 +149,7 @@ __global__ __launch_bounds__(kCsThreads, 1) void transition_stream_kernel(Transi
   static_assert(C % 128 == 0 && C <= 256, "64 + 128 registers of LN(z) and outputs at C = 256");
   constexpr int KS = C / 16, OB = C / 32;
   __shared__ __align__(1024) char smem[T::SMEM];
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
   const int H = p.H, U = H / 32;
@@ -91,13 +157,6 @@ __global__ __launch_bounds__(kCsThreads, 1) void transition_stream_kernel(Transi
   const dma_src_t r2 = dma_src(SWIGLU ? p.w2 : p.w1, (uint32_t)H * C * 2u);
   const dma_src_t r3 = dma_src(p.w3, (uint32_t)H * C * 2u);
 
-  // (each address is computed where it is used from a lane number the compiler cannot hoist: the
-  // loop has no registers left to keep them in)
-  auto fresh_lane = [&]() {
-    int l = lane;
-    __asm__ volatile("" : "+v"(l));
-    return l;
-  };
   // Weight loads: 8 rows of 128 bytes (64 k) per instruction of W1 / W2, 16 rows of 64 bytes (32
   // units) of W3; the 16-byte pieces of a row XOR-swizzled so that a fragment read (32 rows, one
   // piece) covers the banks evenly.
@@ -132,8 +191,7 @@ __global__ __launch_bounds__(kCsThreads, 1) void transition_stream_kernel(Transi
     load12(0);
 
     // 1. The wave's z into its LDS rows, the 16-byte pieces of a row XOR-swizzled by its cell; the
-    // accumulators start from it (the residual); LayerNorm in place, 1 KB at a time in a rolled loop
-    // (straight-line code that runs once per tile is bound by its instruction fetches); fragments.
+    // accumulators start from it (the residual); LayerNorm in place; fragments.
     half8 nf[KS];
     f32x16 o[OB];
     {
@@ -144,55 +202,19 @@ __global__ __launch_bounds__(kCsThreads, 1) void transition_stream_kernel(Transi
         const int c = i * CPI + cl;
         dma16(dz, lds0 + (uint32_t)(zs - smem) + i * 1024, (uint32_t)(c * (2 * C) + 16 * (l0 ^ (c & (LPC - 1)))), 0);
       }
-      float g[8], bb[8];
-#pragma unroll
-      for (int e = 0; e < 8; e++) {
-        g[e] = p.ln_w[8 * l0 + e];
-        bb[e] = p.ln_b[8 * l0 + e];
-      }
       wait_vm(0);
-      {
-        const char* zr = zs + (l & 31) * (2 * C) + 8 * (l >> 5);
 #pragma unroll
-        for (int ob = 0; ob < OB; ob++)
+      for (int ob = 0; ob < OB; ob++)
 #pragma unroll
-          for (int q = 0; q < 4; q++) {
-            const half4 v = *reinterpret_cast<const half4*>(zr + 16 * ((4 * ob + q) ^ (l & (LPC - 1))));
+        for (int q = 0; q < 4; q++) {
+          const half4 v = *reinterpret_cast<const half4*>(acc_piece<C>(zs, l, ob, q));
 #pragma unroll
-            for (int e = 0; e < 4; e++) o[ob][4 * q + e] = (float)v[e];
-          }
-      }
-      cs_lds_fence();
-#pragma unroll 4
-      for (int i = 0; i < NKB; i++) {
-        char* piece = zs + i * 1024 + cl * (2 * C) + 16 * (l0 ^ ((i * CPI + cl) & (LPC - 1)));
-        const half8 x = *reinterpret_cast<const half8*>(piece);
-        const half2v one = {(half_t)1.0f, (half_t)1.0f};
-        const float s0 = __builtin_amdgcn_fdot2(half2v{x[2], x[3]}, one,
-                                                __builtin_amdgcn_fdot2(half2v{x[0], x[1]}, one, 0.f, false), false);
-        const float s1 = __builtin_amdgcn_fdot2(half2v{x[6], x[7]}, one,
-                                                __builtin_amdgcn_fdot2(half2v{x[4], x[5]}, one, 0.f, false), false);
-        const float mean = lane_sum<LPC>(s0 + s1) * (1.0f / C);
-        float q0 = 0.f, q1 = 0.f, d[8];
-#pragma unroll
-        for (int e = 0; e < 8; e++) d[e] = (float)x[e] - mean;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          q0 += d[e] * d[e];
-          q1 += d[e + 4] * d[e + 4];
+          for (int e = 0; e < 4; e++) o[ob][4 * q + e] = (float)v[e];
         }
-        const float rstd = rsqrtf(lane_sum<LPC>(q0 + q1) * (1.0f / C) + p.eps);
-        half8 v;
-#pragma unroll
-        for (int e = 0; e < 8; e++) v[e] = (half_t)(d[e] * rstd * g[e] + bb[e]);
-        *reinterpret_cast<half8*>(piece) = v;
-      }
       cs_lds_fence();
-#pragma unroll
-      for (int k = 0; k < KS; k++)
-        nf[k] = *reinterpret_cast<const half8*>(zs + (l & 31) * (2 * C) + 16 * ((2 * k + (l >> 5)) ^ (l & (LPC - 1))));
-#pragma unroll
-      for (int k = 0; k < KS; k++) pin(nf[k]);
+      ln_rows_lds<C>(zs, p.ln_w, p.ln_b, p.eps);
+      cs_lds_fence();
+      rows_to_frags<C>(zs, nf);
     }
     __syncthreads();  // every wave's rows are read: the ring takes their place
     load3(0);
@@ -298,7 +320,6 @@ __global__ __launch_bounds__(kCsThreads, 1) void transition_stream_kernel(Transi
     // 3. Rounded once, through the wave's LDS rows, out as whole cell rows.
     {
       const int l = fresh_lane();
-      char* zr = zs + (l & 31) * (2 * C) + 8 * (l >> 5);
 #pragma unroll
       for (int ob = 0; ob < OB; ob++)
 #pragma unroll
@@ -306,7 +327,7 @@ __global__ __launch_bounds__(kCsThreads, 1) void transition_stream_kernel(Transi
           half4 v;
 #pragma unroll
           for (int e = 0; e < 4; e++) v[e] = (half_t)o[ob][4 * q + e];
-          *reinterpret_cast<half4*>(zr + 16 * ((4 * ob + q) ^ (l & (LPC - 1)))) = v;
+          *reinterpret_cast<half4*>(acc_piece<C>(zs, l, ob, q)) = v;
         }
       cs_lds_fence();
       const rsrc_t ro = make_rsrc_n(p.out + (nv ? cell0 * C : 0), (uint32_t)nv * C * 2u);
@@ -319,6 +340,227 @@ __global__ __launch_bounds__(kCsThreads, 1) void transition_stream_kernel(Transi
     }
     __syncthreads();  // the rows are the next tile's ring slots
   }
+}
+
+// ---- emit and gate: out = [z +] (LN_mix(x) We^T) * sigmoid(LN_in(z) Wg^T) [* mask] ------------------
+// One launch in place of the transposing LayerNorm of x and the dual GEMM, which wrote and read LN(x) and
+// read a kept LN(z): x and z are read once, both LayerNorms happen on the way into the fragments, z stays in
+// registers (in accumulator order) for the residual. Bound by memory and latency phases: a workgroup loads x
+// (its ~16,000 cycles at the chip's rate), then z, normalises (~10,000), multiplies (8 blocks of ~3,000) and
+// stores. Two workgroups of 4 waves per CU, each with its own weight ring, run these phases against each
+// other; one of 8 waves made the update 499 us at L=476 instead of 457 and 116 instead of 110 at L=238.
+// Traced, the two launches against this one: L=238 15.1 + 42.7 -> 39.9 us, L=476 64.7 + 149.5 -> 113.4 us (348
+// MB of x, z and out: 3.1 TB/s).
+template <int C>
+struct CsEmitGeo {
+  static constexpr int WB = 32 * C * 2, WSB = 2 * WB;       // 32 outputs of We, of Wg; a ring slot holds both
+  static constexpr int NL = WSB / 1024 / kEmWaves;          // 1 KB loads per wave and slot
+  static constexpr int ZW = kCsCells * C * 2;               // a wave's x, then z, then output rows
+  static constexpr int OFFZ = 4 * C * 4;                    // behind the LayerNorm parameters; both ring slots
+  static constexpr int SMEM0 = OFFZ + 2 * WSB, SMEM1 = OFFZ + kEmWaves * ZW;  // take their place
+  static constexpr int SMEM = SMEM0 > SMEM1 ? SMEM0 : SMEM1;
+  static_assert(2 * SMEM <= 160 * 1024, "LDS: two workgroups per CU");
+};
+
+template <int C, bool MASK, bool RES>
+__global__ __launch_bounds__(64 * kEmWaves, 2) void emit_stream_kernel(EpilogueArgs p) {
+  using T = CsEmitGeo<C>;
+  constexpr int KS = C / 16, OB = C / 32, LPC = C / 8, CPI = 64 / LPC, NKB = T::ZW / 1024;
+  static_assert(OB % 2 == 0 && C % (64 * kEmWaves) == 0, "output blocks in pairs; whole parameter loads");
+  __shared__ __align__(1024) char smem[T::SMEM];
+  float* lnp = reinterpret_cast<float*>(smem);  // LN_mix w, b, LN_in w, b
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+  const int L = p.L;
+  // this wave's unit: 32 cells (bi, i, pos0 ..) of one pair row; nv of them inside the row. The XCD-aware
+  // order gives neighbouring units, which share lines of x, one L2.
+  const int u = xcd_remap(blockIdx.x, gridDim.x) * kEmWaves + wave, bl = u / p.tiles_per_line;
+  const int pos0 = (u - bl * p.tiles_per_line) * kCsCells, bi = bl / L, i = bl - bi * L;
+  const bool live = bi < p.B;
+  const int nv = !live ? 0 : L - pos0 < kCsCells ? L - pos0 : kCsCells;
+  const size_t cell0 = live ? ((size_t)bi * L + i) * L + pos0 : 0;
+  const int zoff = T::OFFZ + wave * T::ZW;
+  char* zs = smem + zoff;
+
+  // 1. x: channel rows of 32 cells (64 bytes) into the wave's LDS, transposing reads into fragments,
+  // LayerNorm in registers; z takes x's place meanwhile.
+  half8 nx[KS], nz[KS];
+  half4 zo[OB][4];  // z, then the output, in accumulator order
+  float mv = 1.f;
+  {
+    const int l = fresh_lane();
+    const bool okx = live && pos0 + 8 * (l & 3) < p.ldx;
+    const uint32_t xo = okx ? (uint32_t)((size_t)(l >> 2) * L * p.ldx + 8 * (l & 3)) * 2u : kOOB;
+    const half_t* xb = p.x + (((size_t)(live ? bi : 0) * C) * L + (live ? i : 0)) * p.ldx + (live ? pos0 : 0);
+#pragma unroll 4
+    for (int q = 0; q < C / 16; q++)
+      dma16(dma_src(xb + (size_t)16 * q * L * p.ldx, (uint32_t)kBufRange), lds0 + zoff + q * 1024, xo, 0);
+    for (int c = threadIdx.x; c < C; c += 64 * kEmWaves) {
+      lnp[c] = p.ln_mix_w[c];
+      lnp[C + c] = p.ln_mix_b[c];
+      lnp[2 * C + c] = p.ln_in_w[c];
+      lnp[3 * C + c] = p.ln_in_b[c];
+    }
+    if constexpr (MASK) mv = (l & 31) < nv ? (float)p.mask[cell0 + (l & 31)] : 0.f;
+  }
+  wait_vm(0);
+  __syncthreads();  // the parameters are in LDS
+  {
+    const int l = fresh_lane(), h = l >> 5, n0 = 16 * ((l >> 4) & 1), j = l & 15;
+    const half_t* xs = reinterpret_cast<const half_t*>(zs);
+    float s = 0.f, q = 0.f;
+#pragma unroll
+    for (int k = 0; k < KS; k++) {
+      const half4 lo = ds_read_tr16x4(xs + (16 * k + 8 * h + (j >> 2)) * kCsCells + n0 + 4 * (j & 3));
+      const half4 hi = ds_read_tr16x4(xs + (16 * k + 8 * h + 4 + (j >> 2)) * kCsCells + n0 + 4 * (j & 3));
+      nx[k] = half8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    }
+#pragma unroll
+    for (int k = 0; k < KS; k++) pin(nx[k]);
+    {
+      const dma_src_t dz = dma_src(p.z + cell0 * C, (uint32_t)nv * C * 2u);
+      const int l0 = l & (LPC - 1), cl = l / LPC;
+#pragma unroll 4
+      for (int t = 0; t < NKB; t++) {
+        const int c = t * CPI + cl;
+        dma16(dz, lds0 + zoff + t * 1024, (uint32_t)(c * (2 * C) + 16 * (l0 ^ (c & (LPC - 1)))), 0);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < KS; k++) dot2_moments(nx[k], s, q);
+    s += __shfl_xor(s, 32);
+    q += __shfl_xor(q, 32);
+    float rstd, shift;
+    ln_scale_shift(s, q, 1.0f / C, p.eps_mix, rstd, shift);
+#pragma unroll
+    for (int k = 0; k < KS; k++) {
+      const f32x4* w = reinterpret_cast<const f32x4*>(lnp + 16 * k + 8 * h);
+      const f32x4* b = reinterpret_cast<const f32x4*>(lnp + C + 16 * k + 8 * h);
+      const f32x4 w0 = w[0], w1 = w[1], b0 = b[0], b1 = b[1];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        nx[k][e] = ln_value(nx[k][e], rstd, shift, w0[e], b0[e]);
+        nx[k][e + 4] = ln_value(nx[k][e + 4], rstd, shift, w1[e], b1[e]);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < KS; k++) pin(nx[k]);
+  }
+  wait_vm(0);
+  if constexpr (RES) {
+    const int l = fresh_lane();
+#pragma unroll
+    for (int ob = 0; ob < OB; ob++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) zo[ob][q] = *reinterpret_cast<const half4*>(acc_piece<C>(zs, l, ob, q));
+    cs_lds_fence();
+  }
+  ln_rows_lds<C>(zs, lnp + 2 * C, lnp + 3 * C, p.eps_in);
+  cs_lds_fence();
+  rows_to_frags<C>(zs, nz);
+  __syncthreads();  // every wave's rows are read: the ring takes their place
+
+  // 2. The outputs, 32 at a time: both products, the gate. The next block's weights arrive meanwhile.
+  const dma_src_t re = dma_src(p.w_emit, C * C * 2u), rg = dma_src(p.w_gate, C * C * 2u);
+  auto load_w = [&](int ob) {
+    const uint32_t dst = lds0 + T::OFFZ + (ob & 1) * T::WSB;
+    const int l = fresh_lane();
+    const uint32_t l1 = (uint32_t)(l >> 3) * (C * 2), x1 = 16u * (uint32_t)((l & 7) ^ (l >> 4));
+#pragma unroll
+    for (int t = 0; t < T::NL; t++) {
+      constexpr int N1 = T::WB / 1024;
+      const int q = wave * T::NL + t, m = q / N1, qm = q % N1, st = qm / 4, rq = qm % 4;
+      dma16(m ? rg : re, dst + q * 1024, l1 + (x1 ^ (64u * (rq & 1))), (uint32_t)(32 * ob + 8 * rq) * (C * 2) + st * 128);
+    }
+  };
+  load_w(0);
+  wait_vm(0);
+  __syncthreads();
+  auto block = [&](int ob, half4 (&zb)[4]) {
+    if (ob + 1 < OB) load_w(ob + 1);
+    const int l = fresh_lane(), s1 = T::OFFZ + (ob & 1) * T::WSB + (l & 31) * 128 + 16 * ((l >> 5) ^ ((l >> 1) & 7));
+    auto frag = [&](int q) {
+      const int k = q >> 1, m = q & 1;
+      return *reinterpret_cast<const half8*>(smem + T::OFFZ + ((s1 - T::OFFZ) ^ (32 * (k & 3))) + m * T::WB + (k >> 2) * 4096);
+    };
+    half8 w[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) w[q] = frag(q);
+    f32x16 d1, d2;
+#pragma unroll
+    for (int e = 0; e < 16; e++) d1[e] = d2[e] = 0.f;
+#pragma unroll
+    for (int q = 0; q < 2 * KS; q += 2) {
+      d1 = mfma32(w[q & 3], nx[q / 2], d1);
+      d2 = mfma32(w[(q + 1) & 3], nz[q / 2], d2);
+      if (q + 4 < 2 * KS) {
+        w[q & 3] = frag(q + 4);
+        w[(q + 1) & 3] = frag(q + 5);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        float v = d1[4 * q + e] * sigmoid_from_t(d2[4 * q + e] * kNegLog2e);
+        if constexpr (MASK) v *= mv;
+        if constexpr (RES) v += (float)zb[q][e];
+        __asm__ volatile("" : "+v"(v));  // fp32 then fp16 at every position
+        zb[q][e] = (half_t)v;
+      }
+    wait_vm(0);
+    __syncthreads();
+  };
+#pragma unroll 1
+  for (int ob = 0; ob < OB; ob += 2) {
+    block(ob, zo[0]);
+    block(ob + 1, zo[1]);
+    // the pieces turn by two blocks, so that the loop body names fixed registers
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const half4 t0 = zo[0][q], t1 = zo[1][q];
+#pragma unroll
+      for (int b = 0; b + 2 < OB; b++) zo[b][q] = zo[b + 2][q];
+      zo[OB - 2][q] = t0;
+      zo[OB - 1][q] = t1;
+    }
+  }
+
+  // 3. Out through the wave's LDS rows as whole cell rows.
+  {
+    const int l = fresh_lane();
+#pragma unroll
+    for (int ob = 0; ob < OB; ob++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) *reinterpret_cast<half4*>(acc_piece<C>(zs, l, ob, q)) = zo[ob][q];
+    cs_lds_fence();
+    const rsrc_t ro = make_rsrc_n(p.out + cell0 * C, (uint32_t)nv * C * 2u);
+    const int l0 = l & (LPC - 1), cl = l / LPC;
+#pragma unroll 4
+    for (int t = 0; t < NKB; t++) {
+      const half8 v = *reinterpret_cast<const half8*>(zs + t * 1024 + cl * (2 * C) + 16 * (l0 ^ ((t * CPI + cl) & (LPC - 1))));
+      bstore16(ro, (uint32_t)(t * 1024 + l * 16), v);
+    }
+  }
+}
+
+hipError_t launch_emit_stream(const EpilogueArgs& a, hipStream_t s) {
+  EpilogueArgs e = a;
+  e.tiles_per_line = (a.L + kCsCells - 1) / kCsCells;
+  const long long units = (long long)a.B * a.L * e.tiles_per_line, nt = (units + kEmWaves - 1) / kEmWaves;
+  if (nt * kEmWaves > 0x7fffffffLL) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)nt), blk(64 * kEmWaves);
+  const bool m = a.out_mask && a.mask;
+  if (m && a.residual)
+    ESM_LAUNCH((emit_stream_kernel<256, true, true>), grid, blk, 0, s, e);
+  else if (m)
+    ESM_LAUNCH((emit_stream_kernel<256, true, false>), grid, blk, 0, s, e);
+  else if (a.residual)
+    ESM_LAUNCH((emit_stream_kernel<256, false, true>), grid, blk, 0, s, e);
+  else
+    ESM_LAUNCH((emit_stream_kernel<256, false, false>), grid, blk, 0, s, e);
+  return hipGetLastError();
 }
 
 hipError_t launch_transition_stream(const TransitionArgs& a, int C, int cus, hipStream_t s) {

@@ -178,6 +178,30 @@ def test_transition_256_h1024_across_line_tiles(gpu_lib, pkg, L, swiglu):
     _bar(out, ref, z)
 
 
+@pytest.mark.parametrize("B,L", [(1, 64), (1, 65), (2, 45), (1, 97), (3, 33), (1, 160)])
+@pytest.mark.parametrize("outgoing", [True, False])
+@pytest.mark.parametrize("residual,out_mask", [(True, False), (False, True), (True, True), (False, False)])
+def test_tmu_256_emit_forms(gpu_lib, pkg, B, L, outgoing, residual, out_mask):
+    # the cell-stationary emit / gate kernel from its first size on (64 is the last of the other form), with
+    # partial units in every row, a partial last workgroup, and each form of its output
+    C = 256
+    p = _weights(L + B, C, outgoing)
+    mod = pkg.trimul.TriMul.from_weights(p, out_mask=out_mask)
+    z = torch.randn(B, L, L, C, generator=torch.Generator().manual_seed(L)).half()
+    m = _mask(L + 5, B, L, "random")
+    upd = mod(z.to(DEV), m.to(DEV), residual=residual)
+    with torch.no_grad():
+        ref = tmu.trimul(z.float(), m.float(), p, outgoing)
+    if out_mask:
+        ref = ref * m.float().unsqueeze(-1)
+    rms = float(ref.pow(2).mean().sqrt())
+    err = float((upd.cpu().float() - (ref + z.float() if residual else ref)).abs().max())
+    # 1e-2 RMS of the update as elsewhere, and half an fp16 ulp of the largest output with the residual in it
+    assert err <= 1e-2 * rms + (2 ** -9 if residual else 0.0), (err, rms)
+    again = mod(z.to(DEV), m.to(DEV), residual=residual)
+    assert torch.equal(again, upd)
+
+
 @pytest.mark.parametrize("B,L,H", [(1, 129, 32), (2, 91, 64), (1, 129, 96), (1, 128, 128), (1, 181, 160),
                                    (1, 257, 128)])
 @pytest.mark.parametrize("swiglu", [True, False])
