@@ -296,6 +296,17 @@ static bool stream_emit(int C, int B, int L) {
   return C == 256 && 2LL * B * L * ((L + 31) / 32) > cu_count();
 }
 
+// The projection with its LayerNorm in one launch, instead of a LayerNorm pass and the weight-stationary GEMM
+// (whose LN(z) the emit step then has to form by itself), when its workgroups (16 operand rows x 8 k; two per
+// CU at a time) fill their last round to four fifths or run for more than two rounds. Whole update, us, two
+// launches / one: L = 200 (325 of 512 places) 88.9 / 90.9, L = 238 (450) 115 / 109, L = 260 (561: a second
+// round for 49) 146 / 156, L = 340 (946 of 1,024) 230 / 216, L = 384 (1,152) 283 / 275, L = 476 462 / 434; with
+// a mask L = 238 119 / 113, L = 476 485 / 441.
+static bool stream_project(int C, int B, int L) {
+  const long long slots = 2LL * cu_count(), n = (long long)B * ((L + 15) / 16) * ((L + 7) / 8);
+  return stream_emit(C, B, L) && (n > 2 * slots || 5 * n >= 4 * slots * ((n + slots - 1) / slots));
+}
+
 // The wide path of tmu_forward (C = c, a multiple of 128 other than 128, up to 512): five
 // launches in the workspace planes a | b | x | n (x / 256 as in the narrow path):
 //   n = LN_in(z) (cell-major)  ->  a, b = gate(n W^T) (channel-major, GATE_CM)  ->  x = a b^T
@@ -316,34 +327,42 @@ static int tmu_forward_wide(const esm_half* z, const esm_half* mask, const float
   half_t* wx = wb + a256;
   half_t* wn = wx + a256;
   const float kScale = 1.0f / 256.0f;
-  hipError_t e = esm::launch_ln_rows(z, nullptr, false, ln_in_w, ln_in_b, ln_in_eps, wn, ncell, C, st);
-  if (e != hipSuccess) return hip_status(e, "tmu_forward ln_rows launch");
-  esm::WideArgs g{};
-  g.a1 = wn;
-  g.w1 = H(w_bundle);                       // signal rows [s_a | s_b]
-  g.w2 = H(w_bundle) + (size_t)2 * c * C;   // gate rows [g_a | g_b]
-  g.K = C;
-  g.N = 2 * c;
-  g.B = B;
-  g.L = L;
-  g.tiles_per_line = (L + 127) / 128;
-  g.transpose = outgoing ? 0 : 1;
-  g.mask = mask ? H(mask) : nullptr;
-  g.plane_a = wa;
-  g.plane_b = wb;
-  g.c = c;
-  g.ld = ld;
   // K = C <= 256 runs the weight-stationary GEMM, which writes a, b in the fragment layout
   // (the contraction then reads each operand fragment straight into registers)
   const bool frag = C <= 256;
-  if (frag) {
-    g.frag = 1;
-    g.rbn = (L + 31) / 32;
-    g.kbn = (L + 15) / 16;
+  hipError_t e;
+  if (stream_project(C, B, L)) {
+    esm::ProjectArgs pa{H(z), mask ? H(mask) : nullptr, ln_in_w, ln_in_b, ln_in_eps, H(w_bundle), wa, wb, B, L, ld,
+                        outgoing ? 0 : 1, 0, 0, 1, (L + 31) / 32, (L + 15) / 16};
+    e = esm::launch_project_stream(pa, st);
+    if (e != hipSuccess) return hip_status(e, "tmu_forward gate launch");
+  } else {
+    e = esm::launch_ln_rows(z, nullptr, false, ln_in_w, ln_in_b, ln_in_eps, wn, ncell, C, st);
+    if (e != hipSuccess) return hip_status(e, "tmu_forward ln_rows launch");
+    esm::WideArgs g{};
+    g.a1 = wn;
+    g.w1 = H(w_bundle);                       // signal rows [s_a | s_b]
+    g.w2 = H(w_bundle) + (size_t)2 * c * C;   // gate rows [g_a | g_b]
+    g.K = C;
+    g.N = 2 * c;
+    g.B = B;
+    g.L = L;
+    g.tiles_per_line = (L + 127) / 128;
+    g.transpose = outgoing ? 0 : 1;
+    g.mask = mask ? H(mask) : nullptr;
+    g.plane_a = wa;
+    g.plane_b = wb;
+    g.c = c;
+    g.ld = ld;
+    if (frag) {
+      g.frag = 1;
+      g.rbn = (L + 31) / 32;
+      g.kbn = (L + 15) / 16;
+    }
+    if (esm::wide_gemm_blocks(g) > 0x7fffffffLL) return fail(ESM_ERR_SHAPE, "tmu_forward: too many tiles");
+    e = esm::launch_wide_gemm(g, esm::kWideGateCM, st, cu_count());
+    if (e != hipSuccess) return hip_status(e, "tmu_forward gate launch");
   }
-  if (esm::wide_gemm_blocks(g) > 0x7fffffffLL) return fail(ESM_ERR_SHAPE, "tmu_forward: too many tiles");
-  e = esm::launch_wide_gemm(g, esm::kWideGateCM, st, cu_count());
-  if (e != hipSuccess) return hip_status(e, "tmu_forward gate launch");
   esm::ContractArgs ca{wa, wb, wx, B * c, L, ld, ld, kScale, frag ? 1 : 0};
   e = esm::launch_contract(ca, st);
   if (e != hipSuccess) return hip_status(e, "tmu_forward contract launch");

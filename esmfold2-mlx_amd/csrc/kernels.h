@@ -209,6 +209,8 @@ hipError_t launch_q8_linear(const Q8Args& a, hipStream_t s);
 // gate f <-> column 160 (f / 80) + f % 80, up f <-> that + 80 (N a multiple of 160).
 constexpr int kQ8SwigluHalf = 80;
 hipError_t launch_transition(const TransitionArgs& a, int grid, hipStream_t s);
+// The projection step at C = c = 256 with its LayerNorm, a and b in FragLayout (a.rbn, a.kbn set).
+hipError_t launch_project_stream(const ProjectArgs& a, hipStream_t s);
 // The emit / gate step at C = c = 256 with both LayerNorms (a.ntiles, a.tiles_per_line are set by the launcher).
 hipError_t launch_emit_stream(const EpilogueArgs& a, hipStream_t s);
 // The whole transition at C = 256, H a multiple of 32 (a.ntiles is set by the launcher).

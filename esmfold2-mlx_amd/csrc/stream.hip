@@ -342,6 +342,178 @@ __global__ __launch_bounds__(kCsThreads, 1) void transition_stream_kernel(Transi
   }
 }
 
+// ---- projection: a, b = (LN(z) Ws^T) * sigmoid(LN(z) Wg^T) [* mask], in FragLayout ---------------------
+// One launch in place of the LayerNorm pass and the weight-stationary GEMM. No single limit: at L=476 its 160
+// us hold ~62 us of vector work (the gates' exp and rcp above all), ~26 us of MFMAs and 68 us of memory
+// traffic, and leaving any one of them out saved 20 to 60 us, so what it loses is overlap. Tried on top and not
+// faster: the gate of a block between the products of the next one (100 us for the update at L=238 either
+// way), and 8 waves per workgroup with a ring of three slots (440 us against 414 at L=476).
+template <int C>
+struct CsProjGeo {
+  static constexpr int WB = 32 * C * 2, WSB = 2 * WB;       // 32 signal rows and their gate rows: a ring slot
+  static constexpr int NL = WSB / 1024 / kEmWaves;
+  static constexpr int ZW = kCsCells * C * 2;
+  static constexpr int OFFS = 2 * WSB > kEmWaves * ZW ? 2 * WSB : kEmWaves * ZW;  // z rows, then the ring; then staging
+  static constexpr int STG = 32 * 256;                      // 32 channels x 16 operand rows x 8 k
+  static constexpr int SMEM = OFFS + 2 * STG;               // (the LayerNorm parameters lie in the staging's place)
+  static_assert(2 * SMEM <= 160 * 1024 && 2 * C * 4 <= 2 * STG, "LDS: two workgroups per CU");
+};
+
+// A workgroup takes 16 operand rows x 8 k, a wave four of the rows: its cells c = 8 dr + dc are the
+// rows of D[cell][channel], so a lane ends with 4 consecutive k of one channel and row.
+template <int C, bool MASK>
+__global__ __launch_bounds__(64 * kEmWaves, 2) void project_stream_kernel(ProjectArgs p) {
+  using T = CsProjGeo<C>;
+  constexpr int KS = C / 16, NB = 2 * C / 32, LPC = C / 8, CPI = 64 / LPC, NKB = T::ZW / 1024;
+  static_assert(C % (64 * kEmWaves) == 0, "whole parameter loads");
+  __shared__ __align__(1024) char smem[T::SMEM];
+  float* lnp = reinterpret_cast<float*>(smem + T::OFFS);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+  const int L = p.L;
+  const int nr = (L + 15) / 16, t0 = xcd_remap(blockIdx.x, gridDim.x), bi = t0 / (nr * p.tiles_per_line);
+  const int tt = t0 - bi * nr * p.tiles_per_line, tr = tt / p.tiles_per_line;
+  const int R0 = 16 * tr, K0 = 8 * (tt - tr * p.tiles_per_line);   // first operand row, first k
+  const int row0 = R0 + 4 * wave;
+  const size_t cb = (size_t)bi * L * L + (p.transpose ? (size_t)K0 * L + row0 : (size_t)row0 * L + K0);
+  char* zs = smem + wave * T::ZW;
+  // offset in cells of the wave's cell c from its first one, and whether it lies inside the grid
+  auto coff = [&](int c) { return p.transpose ? (c & 7) * L + (c >> 3) : (c >> 3) * L + (c & 7); };
+  auto cin = [&](int c) { return row0 + (c >> 3) < L && K0 + (c & 7) < L; };
+
+  // 1. z rows into LDS (XOR-swizzled as ln_rows_lds reads them), LayerNorm, fragments; zeros for the cells
+  // past the grid, whose operands are then 0
+  half8 nf[KS];
+  float mv[MASK ? 16 : 1];
+  {
+    const dma_src_t dz = dma_src(p.z + cb * C, (uint32_t)kBufRange);
+    const int l = fresh_lane(), l0 = l & (LPC - 1), cl = l / LPC;
+#pragma unroll 4
+    for (int t = 0; t < NKB; t++) {
+      const int c = t * CPI + cl;
+      dma16(dz, lds0 + wave * T::ZW + t * 1024,
+            cin(c) ? (uint32_t)coff(c) * (2 * C) + 16 * (l0 ^ (c & (LPC - 1))) : kOOB, 0);
+    }
+    for (int c = threadIdx.x; c < C; c += 64 * kEmWaves) {
+      lnp[c] = p.ln_w[c];
+      lnp[C + c] = p.ln_b[c];
+    }
+    if constexpr (MASK) {
+      const rsrc_t rm = make_rsrc(p.mask + cb);
+#pragma unroll
+      for (int e = 0; e < 16; e++) {
+        const int c = 8 * (e >> 2) + 4 * (l >> 5) + (e & 3);
+        mv[e] = h2f(bload2(rm, cin(c) ? (uint32_t)coff(c) * 2u : kOOB));
+      }
+    }
+  }
+  wait_vm(0);
+  __syncthreads();  // the parameters are in LDS
+  ln_rows_lds<C>(zs, lnp, lnp + C, p.eps);
+  cs_lds_fence();
+  rows_to_frags<C>(zs, nf);
+  if (row0 + 4 > L || K0 + 8 > L) {
+    const int l = fresh_lane();
+    const bool in = cin(l & 31);
+#pragma unroll
+    for (int k = 0; k < KS; k++) nf[k] = in ? nf[k] : zero_half8();
+  }
+  __syncthreads();  // every wave's rows are read: the ring takes their place
+
+  // 2. 32 channels at a time (a's, then b's): both products, the gate, the staged tile out as 256-byte
+  // segments (16 rows x 8 k of one channel) while the next block's products run
+  const dma_src_t rw = dma_src(p.w, 4u * C * C * 2u);
+  auto load_w = [&](int ob) {
+    const uint32_t dst = lds0 + (ob & 1) * T::WSB;
+    const int l = fresh_lane();
+    const uint32_t l1 = (uint32_t)(l >> 3) * (C * 2), x1 = 16u * (uint32_t)((l & 7) ^ (l >> 4));
+#pragma unroll
+    for (int t = 0; t < T::NL; t++) {
+      constexpr int N1 = T::WB / 1024;
+      const int q = wave * T::NL + t, m = q / N1, qm = q % N1, st = qm / 4, rq = qm % 4;
+      dma16(rw, dst + q * 1024, l1 + (x1 ^ (64u * (rq & 1))), (uint32_t)(m * 2 * C + 32 * ob + 8 * rq) * (C * 2) + st * 128);
+    }
+  };
+  const size_t plane_h = (size_t)p.rbn * p.kbn * FragLayout::kTileHalfs;
+  const size_t tile_h = ((size_t)(R0 >> 5) * p.kbn + (K0 >> 4)) * FragLayout::kTileHalfs +
+                        (size_t)((R0 & 31) + 32 * ((K0 >> 3) & 1)) * 8;
+  // this wave's share of block ob's staged tile: 2 x 4 channels of 256 bytes
+  auto store = [&](int ob) {
+    const int l = fresh_lane();
+    const char* sg = smem + T::OFFS + (ob & 1) * T::STG;
+    const int ch0 = 32 * ob % C;
+    const rsrc_t ro = make_rsrc((ob < NB / 2 ? p.a : p.b) + ((size_t)bi * C + ch0) * plane_h + tile_h);
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      const int ch = 8 * wave + 4 * t + (l >> 4);
+      bstore16(ro, (uint32_t)(ch * plane_h + 8 * (l & 15)) * 2u,
+               *reinterpret_cast<const half8*>(sg + ch * 256 + 16 * ((l & 15) ^ (ch & 15))));
+    }
+  };
+  load_w(0);
+  wait_vm(0);
+  __syncthreads();
+#pragma unroll 1
+  for (int ob = 0; ob < NB; ob++) {
+    if (ob + 1 < NB) load_w(ob + 1);
+    if (ob > 0) store(ob - 1);
+    const int l = fresh_lane(), s1 = (ob & 1) * T::WSB + (l & 31) * 128 + 16 * ((l >> 5) ^ ((l >> 1) & 7));
+    auto frag = [&](int q) {
+      const int k = q >> 1, m = q & 1;
+      return *reinterpret_cast<const half8*>(smem + (s1 ^ (32 * (k & 3))) + m * T::WB + (k >> 2) * 4096);
+    };
+    constexpr int PF = 6;  // fragments in flight
+    half8 w[PF];
+#pragma unroll
+    for (int q = 0; q < PF; q++) w[q] = frag(q);
+    f32x16 d1, d2;
+#pragma unroll
+    for (int e = 0; e < 16; e++) d1[e] = d2[e] = 0.f;
+#pragma unroll
+    for (int q = 0; q < 2 * KS; q += 2) {
+      d1 = mfma32(nf[q / 2], w[q % PF], d1);
+      d2 = mfma32(nf[q / 2], w[(q + 1) % PF], d2);
+      if (q + PF < 2 * KS) {
+        w[q % PF] = frag(q + PF);
+        w[(q + 1) % PF] = frag(q + PF + 1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    char* sg = smem + T::OFFS + (ob & 1) * T::STG + (l & 31) * 256 + 8 * (l >> 5);
+#pragma unroll
+    for (int dr = 0; dr < 4; dr++) {
+      half4 hv;
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        float v = d1[4 * dr + e] * sigmoidf_fast(d2[4 * dr + e]);
+        if constexpr (MASK) v *= mv[4 * dr + e];
+        __asm__ volatile("" : "+v"(v));  // fp32 then fp16 at every position
+        hv[e] = (half_t)v;
+      }
+      *reinterpret_cast<half4*>(sg + 16 * ((4 * wave + dr) ^ (l & 15))) = hv;
+    }
+    if (ob > 0)
+      wait_vm(2);  // the next block's weights; the two stores behind them may still be on their way
+    else
+      wait_vm(0);
+    __syncthreads();
+  }
+  store(NB - 1);
+}
+
+hipError_t launch_project_stream(const ProjectArgs& a, hipStream_t s) {
+  ProjectArgs t = a;
+  t.tiles_per_line = (a.L + 7) / 8;  // k tiles per row tile
+  const long long nt = (long long)a.B * ((a.L + 15) / 16) * t.tiles_per_line;
+  if (nt > 0x7fffffffLL) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)nt), blk(64 * kEmWaves);
+  if (a.mask)
+    ESM_LAUNCH((project_stream_kernel<256, true>), grid, blk, 0, s, t);
+  else
+    ESM_LAUNCH((project_stream_kernel<256, false>), grid, blk, 0, s, t);
+  return hipGetLastError();
+}
+
 // ---- emit and gate: out = [z +] (LN_mix(x) We^T) * sigmoid(LN_in(z) Wg^T) [* mask] ------------------
 // One launch in place of the transposing LayerNorm of x and the dual GEMM, which wrote and read LN(x) and
 // read a kept LN(z): x and z are read once, both LayerNorms happen on the way into the fragments, z stays in

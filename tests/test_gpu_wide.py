@@ -202,6 +202,22 @@ def test_tmu_256_emit_forms(gpu_lib, pkg, B, L, outgoing, residual, out_mask):
     assert torch.equal(again, upd)
 
 
+@pytest.mark.parametrize("B,L", [(1, 225), (1, 241), (2, 161), (5, 105), (1, 362)])
+@pytest.mark.parametrize("outgoing", [True, False])
+@pytest.mark.parametrize("mask_kind", [None, "random"])
+def test_tmu_256_project_forms(gpu_lib, pkg, B, L, outgoing, mask_kind):
+    # the cell-stationary projection: its smallest grids (L = 225 is the first to fill four fifths of a round),
+    # row and k tiles cut at every remainder, several batch members, more than two rounds
+    C = 256
+    p = _weights(L + B, C, outgoing)
+    z = torch.randn(B, L, L, C, generator=torch.Generator().manual_seed(L)).half()
+    m = _mask(L + 7, B, L, mask_kind)
+    upd = pkg.trimul.TriMul.from_weights(p)(z.to(DEV), None if m is None else m.to(DEV))
+    with torch.no_grad():
+        ref = tmu.trimul(z.float(), torch.ones(B, L, L) if m is None else m.float(), p, outgoing)
+    _bar(upd, ref, torch.zeros_like(ref))
+
+
 @pytest.mark.parametrize("B,L,H", [(1, 129, 32), (2, 91, 64), (1, 129, 96), (1, 128, 128), (1, 181, 160),
                                    (1, 257, 128)])
 @pytest.mark.parametrize("swiglu", [True, False])
