@@ -229,3 +229,31 @@ DEV half8 ln_row128_h(half8 x, const float (&g)[8], const float (&b)[8], float e
   for (int e = 0; e < 8; e++) o[e] = ln_value(x[e], rstd, shift, g[e], b[e]);
   return o;
 }
+
+// --- global memory straight into LDS ---------------------------------------------------------
+// 1 KB of a matrix into LDS, 16 bytes per lane from anywhere in the resource, landing in lane order
+// at a wave-uniform LDS address. Written as assembly because the compiler, which cannot tell a
+// ring's slots apart, waits for every such load in flight before the next LDS read; here the wait is
+// where the slot is handed over (wait_vm and a barrier). Nothing is written to a register.
+// (A uniform value computed in vector registers, an integer division's say, has to be moved to a scalar
+// one by hand for an assembly operand; the waits inside cover that move too.)
+DEV uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+typedef u32x4 dma_src_t;
+DEV dma_src_t dma_src(const void* base, uint32_t bytes) {
+  const uint64_t a = reinterpret_cast<uint64_t>(base);
+  return u32x4{uniform((uint32_t)a), uniform((uint32_t)(a >> 32) & 0xffffu), uniform(bytes), (uint32_t)kBufWord3};
+}
+DEV void dma16(dma_src_t r, uint32_t l, uint32_t off, uint32_t soff) {
+  __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                   :
+                   : "s"(uniform(l)), "v"(off), "s"(r), "s"(uniform(soff))
+                   : "memory");
+}
+#define wait_vm(N) \
+  do { \
+    __builtin_amdgcn_s_waitcnt(0xF70 | (N));  /* vmcnt(N), N < 16 */ \
+    __asm__ volatile("" ::: "memory"); \
+  } while (0)
+DEV uint32_t lds_address(const void* p) {
+  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)p;
+}

@@ -255,7 +255,115 @@ __global__ __launch_bounds__(256, 2) void tmu_contract_frag_kernel(ContractArgs 
   }
 }
 
+// The same contraction on 256 x 256 blocks, one 8-wave workgroup each: the operand tiles of a stage of 32 k (16
+// KB of A, 16 KB of B, whole fragment tiles of 1 KB) go through a ring of four LDS stages that are written by the
+// loads themselves, and each wave reads the fragments of its 128 x 64 outputs from there. Every operand is
+// read from L2 half as often as by the 128 x 128 blocks, which are bound by that traffic once the planes leave
+// the 256 MB cache: 256 channels 131 -> 93 us at L=476 (3.7 TB/s of operands and x), 150 -> 106 at L=512, 411 ->
+// 281 at L=768; 128 channels 53.7 -> 48.7 at L=512, 210 -> 152 at L=768. Same products in the same order:
+// the same bits.
+namespace {
+constexpr int BGT = 512;                 // threads
+constexpr int BGS = 32 * 1024;           // bytes per stage: A (row block, k half), then B
+constexpr int BGN = 4;                   // stages in LDS, three of them in flight
+constexpr int BGR = 256 * 2 + 16;        // output staging row stride (bytes)
+}  // namespace
+
+__global__ __launch_bounds__(BGT, 1) void tmu_contract_block_kernel(ContractArgs p) {
+  constexpr int SMEM = BGN * BGS > 256 * BGR ? BGN * BGS : 256 * BGR;
+  __shared__ __align__(1024) char smem[SMEM];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wr = wave >> 2, wc = wave & 3;
+  const int L = p.L;
+  const int rbn = (L + 31) / 32, kbn = (L + 15) / 16, nb = (rbn + 7) / 8;
+  const int t = xcd_remap(blockIdx.x, gridDim.x);  // a channel's nb^2 blocks share an L2
+  const int ch = t / (nb * nb), rem = t - ch * nb * nb;
+  const int bi = rem / nb, bj = rem - bi * nb;
+  const size_t plane = (size_t)rbn * kbn * FragLayout::kTileHalfs;
+  const uint32_t pbytes = (uint32_t)(plane * 2);
+  const dma_src_t rA = dma_src(p.a + (size_t)ch * plane, pbytes), rB = dma_src(p.b + (size_t)ch * plane, pbytes);
+  const uint32_t lds0 = lds_address(smem);
+  // this wave's share of a stage: row block `wave` of A and of B, both k halves; zeros past L
+  const int lr = lane & 31, lk = 8 * (lane >> 5);
+  const int ra = 8 * bi + wave, rb = 8 * bj + wave;
+  const bool oka = ra < rbn && 32 * ra + lr < L, okb = rb < rbn && 32 * rb + lr < L;
+  const uint32_t va = (uint32_t)ra * kbn * 1024u + lane * 16, vb = (uint32_t)rb * kbn * 1024u + lane * 16;
+  auto load = [&](int s) {
+    const uint32_t dst = lds0 + (s & (BGN - 1)) * BGS + wave * 2048;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      const int kb = 2 * s + h;
+      const bool okk = 16 * kb + lk < L;
+      dma16(rA, dst + h * 1024, oka && okk ? va + kb * 1024u : kOOB, 0);
+      dma16(rB, dst + BGS / 2 + h * 1024, okb && okk ? vb + kb * 1024u : kOOB, 0);
+    }
+  };
+  f32x16 acc[4][2];
+#pragma unroll
+  for (int u = 0; u < 4; u++)
+#pragma unroll
+    for (int v = 0; v < 2; v++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) acc[u][v][e] = 0.f;
+  const int ns = (kbn + 1) / 2;
+#pragma unroll
+  for (int s = 0; s < BGN - 1; s++) load(s);
+  for (int s = 0; s < ns; s++) {
+    wait_vm(4 * (BGN - 2));  // stage s is in LDS (a stage past the end loads zeros, so the count holds)
+    __syncthreads();
+    load(s + BGN - 1);
+    const char* st = smem + (s & (BGN - 1)) * BGS + lane * 16;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      half8 fa[4], fb[2];
+#pragma unroll
+      for (int v = 0; v < 2; v++) fb[v] = *reinterpret_cast<const half8*>(st + BGS / 2 + ((2 * wc + v) * 2 + h) * 1024);
+#pragma unroll
+      for (int u = 0; u < 4; u++) fa[u] = *reinterpret_cast<const half8*>(st + ((4 * wr + u) * 2 + h) * 1024);
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int v = 0; v < 2; v++) acc[u][v] = mfma32(fb[v], fa[u], acc[u][v]);  // D[j][i]
+    }
+  }
+  wait_vm(0);
+  __syncthreads();
+  // lane: i = 32u + lane % 32, j = 32v + 8g + 4 (lane / 32) .. +3
+#pragma unroll
+  for (int u = 0; u < 4; u++)
+#pragma unroll
+    for (int v = 0; v < 2; v++)
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        half4 hv;
+#pragma unroll
+        for (int e = 0; e < 4; e++) hv[e] = (half_t)(acc[u][v][4 * g + e] * p.scale);
+        *reinterpret_cast<half4*>(smem + (128 * wr + 32 * u + lr) * BGR + (64 * wc + 32 * v + acc_row32(4 * g, lane)) * 2) = hv;
+      }
+  __syncthreads();
+  const rsrc_t rX = make_rsrc(p.x + ((size_t)ch * L + 256 * bi) * p.ldx + 256 * bj);
+#pragma unroll 4
+  for (int q = 0; q < 16; q++) {
+    const int row = 32 * wave + 2 * q + (lane >> 5), chunk = lane & 31;
+    const bool ok = 256 * bi + row < L && 256 * bj + 8 * chunk < p.ldx;
+    bstore16(rX, ok ? (uint32_t)(row * p.ldx + 8 * chunk) * 2u : kOOB,
+             *reinterpret_cast<const half8*>(smem + row * BGR + 16 * chunk));
+  }
+}
+
 hipError_t launch_contract(const ContractArgs& a, hipStream_t s) {
+  // 256 x 256 blocks where they cover no more than the 128 x 128 ones (an even count of those per side, four or
+  // more), or a sixth to a fifth more (an odd count, five or more) of planes that the 256 MB cache does not
+  // hold. us, 128 against 256: 256 channels L = 384 (3 per side) 46 / 68, L = 385 75 / 72, L = 513 (5 per
+  // side, 404 MB) 183 / 168; 128 channels L = 256 (2 per side, 128 blocks) 11.3 / 14.0, L = 385 39.6 / 37.1, L = 560
+  // (241 MB) 79 / 96, L = 640 (315 MB) 135 / 116, L = 800 263 / 217.
+  const int nb128 = (a.L + 127) / 128;
+  const double mb = 3.0 * a.batch * a.L * a.L * 2e-6;
+  if (a.frag && (nb128 % 2 == 0 ? nb128 >= 4 : nb128 >= 5 && mb > 256.0)) {
+    const int nb = (a.L + 255) / 256;
+    ESM_LAUNCH(tmu_contract_block_kernel, dim3((unsigned)((long long)a.batch * nb * nb)), dim3(BGT), 0, s, a);
+    return hipGetLastError();
+  }
   if (a.frag) {
     const int nb = ((a.L + 31) / 32 + 3) / 4;
     ESM_LAUNCH(tmu_contract_frag_kernel, dim3((unsigned)((long long)a.batch * nb * nb)), dim3(256), 0, s, a);

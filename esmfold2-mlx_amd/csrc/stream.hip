@@ -13,29 +13,6 @@ constexpr int kCsThreads = 64 * kCsWaves;
 constexpr int kEmWaves = 4;                  // of the kernels that run two workgroups per CU
 constexpr int kCsCells = 32;                 // cells per wave: the columns of one 32x32x16 MFMA
 
-// 1 KB of a matrix into LDS, 16 bytes per lane from anywhere in the resource, landing in lane order
-// at a wave-uniform LDS address. Written as assembly because the compiler, which cannot tell a
-// ring's slots apart, waits for every such load in flight before the next LDS read; here the wait is
-// where the slot is handed over (wait_vm and a barrier). Nothing is written to a register.
-// (A uniform value computed in vector registers, an integer division's say, has to be moved to a scalar
-// one by hand for an assembly operand; the waits inside cover that move too.)
-DEV uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
-typedef u32x4 dma_src_t;
-DEV dma_src_t dma_src(const void* base, uint32_t bytes) {
-  const uint64_t a = reinterpret_cast<uint64_t>(base);
-  return u32x4{uniform((uint32_t)a), uniform((uint32_t)(a >> 32) & 0xffffu), uniform(bytes), (uint32_t)kBufWord3};
-}
-DEV void dma16(dma_src_t r, uint32_t l, uint32_t off, uint32_t soff) {
-  __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                   :
-                   : "s"(uniform(l)), "v"(off), "s"(r), "s"(uniform(soff))
-                   : "memory");
-}
-#define wait_vm(N) \
-  do { \
-    __builtin_amdgcn_s_waitcnt(0xF70 | (N));  /* vmcnt(N), N < 16 */ \
-    __asm__ volatile("" ::: "memory"); \
-  } while (0)
 // Sum over the N = 16 or 32 aligned lanes of a group; every lane gets it.
 template <int N>
 DEV float lane_sum(float v) {
@@ -151,7 +128,7 @@ __global__ __launch_bounds__(kCsThreads, 1) void transition_stream_kernel(Transi
   __shared__ __align__(1024) char smem[T::SMEM];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+  const uint32_t lds0 = lds_address(smem);
   const int H = p.H, U = H / 32;
   const dma_src_t r1 = dma_src(p.w1, (uint32_t)H * C * 2u);
   const dma_src_t r2 = dma_src(SWIGLU ? p.w2 : p.w1, (uint32_t)H * C * 2u);
@@ -369,7 +346,7 @@ __global__ __launch_bounds__(64 * kEmWaves, 2) void project_stream_kernel(Projec
   __shared__ __align__(1024) char smem[T::SMEM];
   float* lnp = reinterpret_cast<float*>(smem + T::OFFS);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+  const uint32_t lds0 = lds_address(smem);
   const int L = p.L;
   const int nr = (L + 15) / 16, t0 = xcd_remap(blockIdx.x, gridDim.x), bi = t0 / (nr * p.tiles_per_line);
   const int tt = t0 - bi * nr * p.tiles_per_line, tr = tt / p.tiles_per_line;
@@ -542,7 +519,7 @@ __global__ __launch_bounds__(64 * kEmWaves, 2) void emit_stream_kernel(EpilogueA
   __shared__ __align__(1024) char smem[T::SMEM];
   float* lnp = reinterpret_cast<float*>(smem);  // LN_mix w, b, LN_in w, b
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+  const uint32_t lds0 = lds_address(smem);
   const int L = p.L;
   // this wave's unit: 32 cells (bi, i, pos0 ..) of one pair row; nv of them inside the row. The XCD-aware
   // order gives neighbouring units, which share lines of x, one L2.

@@ -167,6 +167,34 @@ def test_fragment_layout_path_matches_row_major(gpu_lib, pkg, L, incoming):
     assert torch.isfinite(xf).all()
 
 
+@pytest.mark.parametrize("n,L", [(3, 385), (2, 399), (2, 481), (3, 512), (2, 1000), (110, 641)])
+def test_contract_frag_256_blocks(gpu_lib, pkg, n, L):
+    """The 256 x 256-block contraction (an even count of 128-row blocks per side from four on; L = 641 with 110
+    planes is the odd count past the cache) against the row-major kernel, bit for bit: partial row blocks, odd
+    counts of 16-k steps, and whatever the layout leaves unwritten (rows past L, the 8-k pieces past L) NaN."""
+    lib, K = gpu_lib, pkg.kernels
+    g = torch.Generator(device=DEV).manual_seed(L)
+    ld = K.leading_dim(L)
+    rows, frags = [], []
+    rbn, kbn = (L + 31) // 32, (L + 15) // 16
+    for _ in range(2):
+        t = torch.zeros(n, L, ld, dtype=torch.float16, device=DEV)
+        t[:, :, :L] = torch.randn(n, L, L, generator=g, device=DEV).half()
+        rows.append(t)
+        f = torch.full((n, rbn * 32, kbn * 16), float("nan"), dtype=torch.float16, device=DEV)
+        f[:, :L, :ld] = t
+        # [row block, row, k block, half, 8] -> [row block, k block, half, row, 8]
+        f = f.view(n, rbn, 32, kbn, 2, 8).permute(0, 1, 3, 4, 2, 5).contiguous()
+        assert f[0].numel() == int(lib.tmu_frag_plane_elems(L))
+        frags.append(f)
+    want = K.contract(rows[0], rows[1], L, scale=1 / 256)
+    x = torch.full((n, L, ld), float("nan"), dtype=torch.float16, device=DEV)
+    pkg.capi.check(lib.tmu_contract_frag(frags[0].data_ptr(), frags[1].data_ptr(), x.data_ptr(), n, L, ld, 1 / 256,
+                                         pkg.capi.stream_ptr()))
+    torch.cuda.synchronize()
+    assert torch.equal(x[:, :, :L].view(torch.int16), want[:, :, :L].view(torch.int16))
+
+
 @pytest.mark.parametrize("L", [5, 64, 100])
 @pytest.mark.parametrize("residual", [False, True])
 def test_epilogue_kernel(gpu_lib, pkg, L, residual):
