@@ -856,6 +856,95 @@ int esmc_swiglu(const esm_half* x12, esm_half* y, int M, int F, void* stream) {
   return hip_status(esm::launch_esmc_swiglu(H(x12), H(y), (size_t)M, F, (hipStream_t)stream), "esmc_swiglu launch");
 }
 
+// The pieces of esmc_block's workspace, each 256-byte aligned: qkv, q, k, v, the attention's output, the
+// residual and its LayerNorm between the halves, the gated FFN rows, and the split-K partials of whichever
+// linear runs.
+namespace {
+struct EsmcBlockWs {
+  size_t qkv, q, k, v, o, x_mid, h2, act, parts, parts_bytes, total;
+};
+EsmcBlockWs esmc_block_layout(int M, int D, int F) {
+  EsmcBlockWs w;
+  size_t at = 0;
+  const auto take = [&](size_t bytes) {
+    const size_t here = at;
+    at += (bytes + 255) / 256 * 256;
+    return here;
+  };
+  const size_t md = (size_t)M * D;
+  w.qkv = take(3 * md * 2);
+  w.q = take(md * 2);
+  w.k = take(md * 2);
+  w.v = take(md * 2);
+  w.o = take(md * 2);
+  w.x_mid = take(md * 4);
+  w.h2 = take(md * 2);
+  w.act = take((size_t)M * F * 2);
+  w.parts_bytes = std::max({q8_linear_workspace_bytes(M, D, 3 * D), q8_linear_partials_bytes(M, D, D),
+                            q8_linear_workspace_bytes(M, D, 2 * F), q8_linear_partials_bytes(M, F, D)});
+  w.parts = take(w.parts_bytes);
+  w.total = at;
+  return w;
+}
+}  // namespace
+
+size_t esmc_block_workspace_bytes(int M, int n_heads, int F) {
+  if (M <= 0 || n_heads <= 0 || n_heads * 64 > 4096 || F <= 0 || F % 320 != 0) return 0;
+  return esmc_block_layout(M, n_heads * 64, F).total;
+}
+
+int esmc_block(const float* x, const esm_half* h, const int* sequence_id, const float* q_ln, const float* k_ln,
+               const float* ln2_w, const float* ln2_b, const float* next_w, const float* next_b,
+               const uint8_t* wqkv_qp, const uint32_t* wqkv_sb, const uint8_t* wo_qp, const uint32_t* wo_sb,
+               const uint8_t* w1_qp, const uint32_t* w1_sb, const uint8_t* w2_qp, const uint32_t* w2_sb, float eps,
+               float alpha, float rope_base, float* x_out, esm_half* h_out, float* h_out_fp32, int B, int L,
+               int n_heads, int F, void* workspace, size_t workspace_bytes, void* stream) {
+  if (B < 0 || L < 0 || n_heads <= 0) return fail(ESM_ERR_SHAPE, "esmc_block: B=%d L=%d heads=%d", B, L, n_heads);
+  if (n_heads * 64 > 4096 || F <= 0 || F % 320 != 0)
+    return fail(ESM_ERR_UNSUPPORTED, "esmc_block: heads=%d F=%d (width <= 4096, F a multiple of 320)", n_heads, F);
+  if (!(eps >= 0.f)) return fail(ESM_ERR_SHAPE, "esmc_block: eps must be >= 0");
+  if (B == 0 || L == 0) return ok();
+  const long long m = (long long)B * L;
+  const int D = n_heads * 64;
+  const int wide = std::max(D, F);  // as the linears check their x
+  if (L > 65536 || m * wide * 2 >= (1LL << 31) || (long long)B * n_heads > 65535)
+    return fail(ESM_ERR_SHAPE, "esmc_block: B=%d L=%d heads=%d F=%d too large", B, L, n_heads, F);
+  const int M = (int)m;
+  // everything is checked here, before the first of the launches
+  if (!x || !h || !q_ln || !k_ln || !ln2_w || !next_w || !wqkv_qp || !wqkv_sb || !wo_qp || !wo_sb || !w1_qp || !w1_sb ||
+      !w2_qp || !w2_sb || !x_out || (!h_out == !h_out_fp32) || !workspace)
+    return fail(ESM_ERR_NULL, "esmc_block: NULL pointer (exactly one of h_out, h_out_fp32 is written)");
+  for (const void* q : {(const void*)x, (const void*)h, (const void*)q_ln, (const void*)k_ln, (const void*)wqkv_qp,
+                        (const void*)wqkv_sb, (const void*)wo_qp, (const void*)wo_sb, (const void*)w1_qp,
+                        (const void*)w1_sb, (const void*)w2_qp, (const void*)w2_sb, (const void*)x_out,
+                        (const void*)h_out, (const void*)h_out_fp32})
+    if (!aligned16(q)) return fail(ESM_ERR_ALIGN, "esmc_block: activations, weights and outputs must be 16-byte aligned");
+  const EsmcBlockWs w = esmc_block_layout(M, D, F);
+  if (workspace_bytes < w.total)
+    return fail(ESM_ERR_SHAPE, "esmc_block: workspace of %zu bytes, %zu needed", workspace_bytes, w.total);
+  if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0)
+    return fail(ESM_ERR_ALIGN, "esmc_block: workspace must be 256-byte aligned");
+  char* ws = static_cast<char*>(workspace);
+  const auto half_at = [&](size_t off) { return reinterpret_cast<esm_half*>(ws + off); };
+  esm_half *qkv = half_at(w.qkv), *q = half_at(w.q), *k = half_at(w.k), *v = half_at(w.v), *o = half_at(w.o);
+  float* x_mid = reinterpret_cast<float*>(ws + w.x_mid);
+  float* parts = reinterpret_cast<float*>(ws + w.parts);
+  int splits = 0, rc;
+  if ((rc = q8_linear_packed_ws(h, wqkv_qp, wqkv_sb, qkv, M, D, 3 * D, 64, parts, w.parts_bytes, stream))) return rc;
+  if ((rc = esmc_qk_rope(qkv, q_ln, k_ln, eps, q, k, v, B, L, n_heads, 64, rope_base, stream))) return rc;
+  if ((rc = esmc_attention(q, k, v, sequence_id, o, B, L, n_heads, 64, 0.125f, stream))) return rc;
+  if ((rc = q8_linear_packed_partials(o, wo_qp, wo_sb, parts, w.parts_bytes, &splits, M, D, D, 64, stream))) return rc;
+  if ((rc = esmc_layer_norm_parts(x, parts, splits, alpha, x_mid, ln2_w, ln2_b, eps, half_at(w.h2), nullptr, M, D,
+                                  stream)))
+    return rc;
+  if ((rc = q8_linear_swiglu_packed_ws(half_at(w.h2), w1_qp, w1_sb, half_at(w.act), M, D, 2 * F, 64, parts,
+                                       w.parts_bytes, stream)))
+    return rc;
+  if ((rc = q8_linear_packed_partials(half_at(w.act), w2_qp, w2_sb, parts, w.parts_bytes, &splits, M, F, D, 64, stream)))
+    return rc;
+  return esmc_layer_norm_parts(x_mid, parts, splits, alpha, x_out, next_w, next_b, eps, h_out, h_out_fp32, M, D, stream);
+}
+
 int parcae_step(const float* z, const float* z_init, const float* refined, const float* ln_w, const float* ln_b,
                 float eps, const float* a, const esm_half* b_mat, float* z_out, int B, int L, int C, void* stream) {
   if (B < 0 || L < 0) return fail(ESM_ERR_SHAPE, "parcae_step: B=%d L=%d must be >= 0", B, L);

@@ -120,28 +120,41 @@ class EsmcBlock(nn.Module):
         act = self.w1.swiglu(h2) if self.w1.pair_rows else kernels.esmc_swiglu(self.w1(h2))
         return self.w2.partials(act)
 
+    def run(self, x: torch.Tensor, h: torch.Tensor, sid, res_scale: float, next_w, next_b, x_out: torch.Tensor,
+            out: torch.Tensor) -> None:
+        """The block on x [B, L, D] fp32 and h = LN1(x): x_out = its output, out = the LayerNorm (next_w, next_b)
+        of that (fp16 or fp32). One native call when every linear has its packed layouts (codes of a width that
+        is a multiple of 128, so that their size says which shape they are), else the separate calls."""
+        B, L, D = x.shape
+        lins = (self.wqkv, self.wo, self.w1, self.w2)
+        if (self.w1.pair_rows and not any(m.pair_rows for m in (self.wqkv, self.wo, self.w2)) and B and L
+                and self.F % 320 == 0 and D % 128 == 0 and all(m.codes_packed is not None for m in lins)):
+            kernels.esmc_block(x, h, (self.q_ln, self.k_ln, self.ln2_w, self.ln2_b),
+                               [(m.codes_packed, m.packed) for m in lins], next_w, next_b, EPS, 1.0 / res_scale, B, L,
+                               self.n_heads, self.F, x_out, out, sid)
+            return
+        x_mid, h2 = torch.empty_like(x), torch.empty_like(h)
+        self.attention(x, h, sid, res_scale, x_mid, h2)
+        kernels.esmc_layer_norm(x_mid, next_w, next_b, EPS, y_parts=self.ffn(h2), alpha=1.0 / res_scale, x_out=x_out,
+                                out=out, fp32_out=out.dtype == torch.float32)
+
     def forward(self, x: torch.Tensor, sequence_id=None, res_scale: float = 1.0) -> torch.Tensor:
         """One block on an fp32 residual [B, L, D] (the reference's block_forward, mlx_esmc.py:84-102)."""
         x = x.to(torch.float32).contiguous()
         h = kernels.esmc_layer_norm(x, self.ln1_w, self.ln1_b, EPS)
-        x_mid, h2 = torch.empty_like(x), torch.empty_like(h)
-        self.attention(x, h, _chain_ids(sequence_id, x.device), res_scale, x_mid, h2)
         out = torch.empty_like(x)
-        # out = x_mid + y2 / res_scale (the LN output of this call is not needed)
-        kernels.esmc_layer_norm(x_mid, self.ln1_w, self.ln1_b, EPS, y_parts=self.ffn(h2), alpha=1.0 / res_scale,
-                                x_out=out, out=torch.empty_like(h))
+        # (the LN output of this call is not needed)
+        self.run(x, h, _chain_ids(sequence_id, x.device), res_scale, self.ln1_w, self.ln1_b, out, torch.empty_like(h))
         return out
 
 
 def _chain_ids(sequence_id, device):
-    """int32 [B, L] chain ids for the attention mask, or None when every token may attend to
-    every other (a single chain: the reference skips the mask, mlx_esmc.py:188-191)."""
+    """int32 [B, L] chain ids for the attention mask, or None without any. A single chain's ids are passed on too,
+    where the reference skips the mask (mlx_esmc.py:188-191): to tell would be a wait for the GPU in every
+    call, and the mask then changes no bit."""
     if sequence_id is None:
         return None
-    sid = sequence_id.to(device=device)
-    if bool((sid == sid[:, :1]).all()):
-        return None
-    return sid.to(torch.int32).contiguous()
+    return sequence_id.to(device=device).to(torch.int32).contiguous()
 
 
 class HipEsmc(nn.Module):
@@ -237,19 +250,14 @@ class HipEsmc(nn.Module):
         hs[0] = self.embed[ids]
         sid = _chain_ids(sequence_id, dev)
         h = kernels.esmc_layer_norm(hs[0], self.layers[0].ln1_w, self.layers[0].ln1_b, EPS)
-        h2 = torch.empty_like(h)
-        x_mid = torch.empty(B, L, D, dtype=torch.float32, device=dev)
-        x_last = torch.empty_like(x_mid)
+        x_last = torch.empty(B, L, D, dtype=torch.float32, device=dev)
+        states = hs.unbind(0)
         for i, blk in enumerate(self.layers):
-            blk.attention(hs[i], h, sid, self.res_scale, x_mid, h2)
-            y2 = blk.ffn(h2)
-            if i + 1 < n:  # second residual into hidden_states[i+1], fused with the next input LN
+            if i + 1 < n:  # the output into hidden_states[i+1], fused with the next input LN
                 nxt = self.layers[i + 1]
-                kernels.esmc_layer_norm(x_mid, nxt.ln1_w, nxt.ln1_b, EPS, y_parts=y2, alpha=1.0 / self.res_scale,
-                                        x_out=hs[i + 1], out=h)
+                blk.run(states[i], h, sid, self.res_scale, nxt.ln1_w, nxt.ln1_b, states[i + 1], h)
             else:  # the last block's output is only seen through the final norm (weights only)
-                kernels.esmc_layer_norm(x_mid, self.norm_w, None, EPS, y_parts=y2, alpha=1.0 / self.res_scale,
-                                        x_out=x_last, out=hs[n], fp32_out=True)
+                blk.run(states[i], h, sid, self.res_scale, self.norm_w, None, x_last, states[n])
         return hs
 
     def forward(self, input_ids=None, sequence_id=None, output_hidden_states=True, **_):

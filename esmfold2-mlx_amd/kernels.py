@@ -203,6 +203,43 @@ def esmc_swiglu(x12, out=None):
     return y
 
 
+def _weight(t, name: str, dtype, nbytes: int) -> int:
+    """Device pointer of a module's weight after the checks its separate call makes."""
+    if not (t.is_cuda and t.dtype is dtype and t.is_contiguous()):
+        _dev(t, name, dtype)
+    if t.numel() * t.element_size() < nbytes:
+        raise capi.EsmError(-2, f"{name} too small for this shape")
+    return t.data_ptr()
+
+
+def esmc_block(x, h, norms, linears, next_w, next_b, eps, alpha: float, B: int, L: int, n_heads: int, F: int, x_out,
+               out, sequence_id=None, base: float = 10000.0):
+    """One whole block in one call: x [B*L, D] fp32 and h = LN1(x) fp16 -> ``x_out`` fp32 and ``out`` = the
+    LayerNorm (next_w, next_b) of it, fp16 or fp32 by its dtype. ``norms`` = (q_ln, k_ln, ln2_w, ln2_b),
+    ``linears`` = ((codes, packed) of wqkv, wo, w1 in SwiGLU pair order, w2). Its intermediate rows live in the
+    device's shared scratch; the bits are those of the separate calls."""
+    lib = capi.lib()
+    M, D = B * L, 64 * n_heads
+    _out(x, "x", torch.float32, M * D)
+    _out(h, "h", F16, M * D)
+    _out(x_out, "x_out", torch.float32, M * D)
+    fp32 = out.dtype is torch.float32
+    _out(out, "out", torch.float32 if fp32 else F16, M * D)
+    sid = None if sequence_id is None else _out(sequence_id, "sequence_id", torch.int32, M).data_ptr()
+    ln = [_weight(t, n, torch.float32, 4 * D) for t, n in zip(norms, ("q_ln", "k_ln", "ln2_w", "ln2_b"))]
+    ln.append(_weight(next_w, "w", torch.float32, 4 * D))
+    ln.append(None if next_b is None else _weight(next_b, "b", torch.float32, 4 * D))
+    lin = []
+    for (codes, packed), K, N, n in zip(linears, (D, D, D, F), (3 * D, D, 2 * F, D), ("wqkv", "wo", "w1", "w2")):
+        lin.append(_weight(codes, n + " codes", torch.uint8, N * K))
+        lin.append(_weight(packed, n + " packed", torch.int32, N * K // 16))
+    need = int(lib.esmc_block_workspace_bytes(M, n_heads, F))
+    ws, wp, stream = scratch.take(need, x.device)
+    capi.check(lib.esmc_block(x.data_ptr(), h.data_ptr(), sid, *ln, *lin, float(eps), float(alpha), float(base),
+                              x_out.data_ptr(), None if fp32 else out.data_ptr(), out.data_ptr() if fp32 else None, B,
+                              L, n_heads, F, wp, need, stream))
+
+
 def parcae_step(z, z_init, refined, ln_w, ln_b, eps, a, b_mat, out=None):
     """a * z + LN(z_init + refined) @ B^T: z, z_init, refined [B, L, L, C] fp32; b_mat [C, C] fp16."""
     lib = capi.lib()
@@ -419,6 +456,24 @@ def q8_linear(x, q, s, b, group: int = 64, out=None, workspace=None, packed=None
     else:
         capi.check(lib.q8_linear_ws(x.data_ptr(), q.data_ptr(), s.data_ptr(), b.data_ptr(), sbp, y.data_ptr(), M, K,
                                     N, group, wp, wn, capi.stream_ptr()))
+    return y
+
+
+def q8_linear_packed(x, codes, packed, N: int, group: int = 64):
+    """``q8_linear`` on packed weights alone (``q8_pack_codes`` and ``q8_pack_scales`` of a [N, K] matrix), its
+    split-K partials in the device's shared scratch: the same bits, one call."""
+    lib = capi.lib()
+    _dev(x, "x", F16)
+    M, K = x.shape
+    qp = _weight(codes, "codes", torch.uint8, int(lib.q8_packed_codes_bytes(N, K)))
+    sb = _weight(packed, "packed", torch.int32, int(lib.q8_packed_scales_bytes(N, K)))
+    y = torch.empty(M, N, dtype=F16, device=x.device)
+    need = int(lib.q8_linear_workspace_bytes(M, K, N))
+    if need:
+        ws, wp, stream = scratch.take(need, x.device)
+    else:
+        ws, wp, stream = None, None, capi.stream_ptr()
+    capi.check(lib.q8_linear_packed_ws(x.data_ptr(), qp, sb, y.data_ptr(), M, K, N, group, wp, need, stream))
     return y
 
 

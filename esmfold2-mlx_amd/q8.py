@@ -91,12 +91,14 @@ class Q8Linear(nn.Module):
         return kernels.q8_dequant(self.q, self.scales, self.biases, GROUP)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        sb, qp = self._layouts()
+        if qp is not None and x.dim() == 2 and x.dtype == torch.float16 and x.shape[1] == self.in_features and len(x):
+            return kernels.q8_linear_packed(x.contiguous(), qp, sb, self.out_features, GROUP)
         lead = x.shape[:-1]
         x2 = x.reshape(-1, self.in_features).to(torch.float16).contiguous()
         M = x2.shape[0]
         n = kernels.q8_workspace_bytes(M, self.in_features, self.out_features)
         ws = scratch.get(n, x2.device) if n else None  # split-K partials, only while this call runs
-        sb, qp = self._layouts()
         y = kernels.q8_linear(x2, self.q, self.scales, self.biases, GROUP, workspace=ws, packed=sb, codes=qp)
         y = y.reshape(*lead, self.out_features)
         return y if x.dtype == torch.float16 else y.to(x.dtype)

@@ -49,8 +49,8 @@ def _index(device) -> int:
     return torch.cuda.current_device() if d.index is None else d.index
 
 
-def get(nbytes: int, device=None) -> torch.Tensor:
-    """A uint8 view of ``nbytes`` (>= 1) at a 256-byte aligned address of the device's scratch."""
+def _claim(nbytes: int, device):
+    """(the device's buffer, grown if need be, the current stream on it)."""
     idx = _index(device)
     need = max(int(nbytes), 1) + ALIGN
     stream = torch.cuda.current_stream(idx)
@@ -70,9 +70,21 @@ def get(nbytes: int, device=None) -> torch.Tensor:
                 slot.buf.record_stream(stream)
             slot.stream = stream
         slot.generation += 1
-        buf = slot.buf
+        return slot.buf, stream
+
+
+def get(nbytes: int, device=None) -> torch.Tensor:
+    """A uint8 view of ``nbytes`` (>= 1) at a 256-byte aligned address of the device's scratch."""
+    buf, _ = _claim(nbytes, device)
     off = (-buf.data_ptr()) % ALIGN
     return buf[off:off + max(int(nbytes), 1)]
+
+
+def take(nbytes: int, device=None):
+    """``get`` for one launch: (buffer, 256-byte aligned address in it, raw stream). The caller holds the
+    buffer until its launches are queued."""
+    buf, stream = _claim(nbytes, device)
+    return buf, (buf.data_ptr() + ALIGN - 1) // ALIGN * ALIGN, stream.cuda_stream
 
 
 def generation(device=None) -> int:

@@ -407,6 +407,25 @@ int esmc_attention(const esm_half* q, const esm_half* k, const esm_half* v, cons
 int esmc_swiglu(const esm_half* x12, esm_half* y, int M, int F, void* stream);
 
 /*
+ * One whole ESMC block (mlx_esmc.py:84-102) as its nine launches on the stream, from the block's LayerNormed
+ * input: x' = x + alpha * wo(attention(wqkv(h))), then x_out = x' + alpha * w2(swiglu(w1(LN2(x')))), then the
+ * LayerNorm that follows (the next block's input norm, or the final one): h_out fp16 or h_out_fp32, exactly
+ * one of them. The same bits as the separate calls (q8_linear_packed_ws, esmc_qk_rope, esmc_attention,
+ * q8_linear_packed_partials, esmc_layer_norm_parts, q8_linear_swiglu_packed_ws). x, x_out [B*L, D] fp32, h,
+ * h_out [B*L, D] fp16 (h_out may be h), D = 64 n_heads <= 4096, F a multiple of 320; ln2_b, next_b and sequence_id may
+ * be NULL; the linears by their q8_pack_codes / q8_pack_scales layouts, w1 [2F, D] in SwiGLU pair order.
+ * workspace: esmc_block_workspace_bytes(B*L, n_heads, F) bytes, 256-byte aligned. Every argument is checked
+ * before the first launch.
+ */
+size_t esmc_block_workspace_bytes(int M, int n_heads, int F);
+int esmc_block(const float* x, const esm_half* h, const int* sequence_id, const float* q_ln, const float* k_ln,
+               const float* ln2_w, const float* ln2_b, const float* next_w, const float* next_b,
+               const uint8_t* wqkv_qp, const uint32_t* wqkv_sb, const uint8_t* wo_qp, const uint32_t* wo_sb,
+               const uint8_t* w1_qp, const uint32_t* w1_sb, const uint8_t* w2_qp, const uint32_t* w2_sb, float eps,
+               float alpha, float rope_base, float* x_out, esm_half* h_out, float* h_out_fp32, int B, int L,
+               int n_heads, int F, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * The recycling step around the trunk.
  *
  * parcae_step: z_out = a * z + LN(z_init + refined; ln_w, ln_b, eps) @ B^T on every

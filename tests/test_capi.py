@@ -196,6 +196,31 @@ def test_pair_forward_validates_before_launching(lib):
     assert pair(B=600) == -2                        # B * c beyond the contraction's grid
 
 
+def test_esmc_block_validates_before_launching(lib):
+    P = 1 << 20  # an aligned address that is never read: every call below is refused on the host
+    need = lib.esmc_block_workspace_bytes(10, 4, 320)
+    assert need > 0 and lib.esmc_block_workspace_bytes(10, 4, 384) == 0
+    base = dict(ptrs=[P, P, None] + [P] * 5 + [None] + [P] * 8, eps=1e-5, out=[P, P, None], dims=[1, 10, 4, 320], ws=P,
+                n=need)
+
+    def call(**kw):
+        a = {**base, **kw}
+        return lib.esmc_block(*a["ptrs"], a["eps"], 1.0, 1e4, *a["out"], *a["dims"], a["ws"], a["n"], None)
+
+    for i in [i for i in range(17) if i not in (2, 6, 8)]:  # (ids and LayerNorm biases may be NULL)
+        q = list(base["ptrs"])
+        q[i] = None
+        assert call(ptrs=q) == -1, i
+    assert call(out=[P, P, P]) == -1 and call(out=[P, None, None]) == -1 and call(out=[None, P, None]) == -1
+    assert call(ws=None) == -1 and call(n=need - 1) == -2 and call(ws=P + 16) == -3
+    q = list(base["ptrs"])
+    q[9] = P + 8
+    assert call(ptrs=q) == -3
+    assert call(dims=[1, 10, 4, 384]) == -4 and call(dims=[1, 10, 65, 320]) == -4 and call(dims=[-1, 10, 4, 320]) == -2
+    assert call(dims=[1, 70000, 4, 320]) == -2 and call(eps=-1.0) == -2
+    assert call(dims=[0, 10, 4, 320], ptrs=[None] * 17) == 0
+
+
 def test_sized_forward_refuses_a_small_workspace(lib):
     f, ws = ctypes.c_void_p(4096), ctypes.c_void_p(1 << 20)
     o = [f, f, 1e-5, f, f, f, 1e-5, f, f, 0]

@@ -188,6 +188,28 @@ def test_block_real_width(gpu_lib, pkg):
     assert err <= 1e-2 * float(upd.pow(2).mean().sqrt()), err
 
 
+@pytest.mark.parametrize("B,L,D,F_,H", [(1, 1, 128, 320, 2), (2, 33, 256, 640, 4), (1, 130, 2560, 5120, 40)])
+@pytest.mark.parametrize("chains", [None, 1, 3])
+@pytest.mark.parametrize("fp32_out", [False, True])
+def test_native_block_equals_the_separate_calls(gpu_lib, pkg, B, L, D, F_, H, chains, fp32_out):
+    # the one-call block against the launches made one by one, bit for bit: output, the LayerNorm behind it,
+    # with and without its bias, no ids, a single chain's ids and several chains'
+    blk = _module_block(pkg, _weights(D, F_, seed=L), H)
+    x = (2 * torch.randn(B, L, D, generator=_gen(L))).to(DEV)
+    sid = None if chains is None else (torch.arange(L) * chains // L).expand(B, L).to(DEV, torch.int32).contiguous()
+    h = pkg.kernels.esmc_layer_norm(x, blk.ln1_w, blk.ln1_b, 1e-5)
+    nb = None if fp32_out else blk.ln1_b
+    got_x, got_h = torch.empty_like(x), torch.empty(x.shape, dtype=torch.float32 if fp32_out else torch.float16, device=DEV)
+    before = pkg.scratch.generation(DEV)
+    blk.run(x, h, sid, 1.5, blk.ln1_w, nb, got_x, got_h)
+    assert pkg.scratch.generation(DEV) == before + 1  # one native call
+    x_mid, h2, want_x = torch.empty_like(x), torch.empty_like(h), torch.empty_like(x)
+    blk.attention(x, h, sid if chains == 3 else None, 1.5, x_mid, h2)
+    want_h = pkg.kernels.esmc_layer_norm(x_mid, blk.ln1_w, nb, 1e-5, y_parts=blk.ffn(h2), alpha=1 / 1.5, x_out=want_x,
+                                         fp32_out=fp32_out)
+    assert torch.equal(got_x, want_x) and torch.equal(got_h, want_h)
+
+
 def test_block_graph_replay(gpu_lib, pkg):
     """The block captured as one HIP graph: every replay equals the eager result bit for bit,
     with eager launches of the block between the replays."""
