@@ -253,9 +253,11 @@ __global__ __launch_bounds__(kRopeMaxThreads) void esmc_qk_rope_kernel(EsmcRopeA
 }
 
 // ---- attention ---------------------------------------------------------------------------------
-// One workgroup = 4 waves = 32 queries of one (batch, head). Keys go in passes of LP (256
-// or 512; one pass up to L = 512, any length beyond in several, with an online softmax
-// carrying each wave's running max, sum and O across passes). Per pass wave w takes keys
+// One workgroup = 4 waves = 32 queries of one (batch, head). Keys go in passes of LP = 256 (any
+// length beyond in several, with an online softmax carrying each wave's running max, sum and O
+// across passes; passes of 512 leave room for one workgroup per CU instead of two: 40 heads, L = 512
+// 17.7 -> 12.8 us, L = 1100 71.5 -> 40.6, with two chains, whose other half is skipped, 72.6 -> 32.0).
+// Per pass wave w takes keys
 // [base + KW w, base + KW (w + 1)) (KW = LP / 4): it streams its K and V rows into a private LDS region
 // with buffer loads that write LDS directly, computes S^T = K Q^T for its keys and a
 // softmax partial in fp32 (row max m_w, sum l_w, O_w = P V), and the four partials merge
@@ -277,8 +279,8 @@ DEV half4 tr_read_v(const char* vs, int k0, int n0, int lane) {
   return ds_read_tr16x4(vs + n * 128 + 16 * ((d >> 3) ^ (((n >> 1) & 1) << 2)) + 2 * (d & 7));
 }
 
-template <int NKB>
-__global__ __launch_bounds__(256, NKB <= 8 ? 2 : 1) void esmc_attention_kernel(EsmcAttnArgs p) {
+__global__ __launch_bounds__(256, 2) void esmc_attention_kernel(EsmcAttnArgs p) {
+  constexpr int NKB = 8;  // 32-key blocks per pass
   constexpr int HD = 64, LP = 32 * NKB, KW = LP / 4, KB = KW / 32;  // keys and key blocks per wave
   static_assert(KW % 64 == 0, "whole 64-lane loads of key ids");
   __shared__ __align__(16) char kv_s[4][2 * KW * 128];  // per wave: K rows, then V rows
@@ -318,9 +320,30 @@ __global__ __launch_bounds__(256, NKB <= 8 ? 2 : 1) void esmc_attention_kernel(E
   for (int db = 0; db < HD / 32; db++)
 #pragma unroll
     for (int i = 0; i < 16; i++) o[db][i] = 0.f;
+  // With more than one pass, queries of one chain (any block inside a chain) skip a wave's pass whose keys are
+  // all of other chains: every probability there is 0. The next pass's key ids are loaded a pass ahead.
+  const int qsid0 = __builtin_amdgcn_readfirstlane(qsid);
+  const bool one_chain = has_sid && L > LP && __all(qrow >= L || qsid == qsid0);
+  auto key_ids = [&](int base, int (&id)[KW / 64]) {
+#pragma unroll
+    for (int i = 0; i < KW / 64; i++)
+      id[i] = __builtin_amdgcn_raw_buffer_load_b32(rs, (int)((uint32_t)(base + KW * wave + 64 * i + lane) * 4u), 0, 0);
+  };
+  int kid[KW / 64], kid_next[KW / 64];
+  if (one_chain) key_ids(0, kid_next);
   for (int base = 0; base < L; base += LP) {
     const int key0 = base + KW * wave;
-    const bool live = key0 < L;  // wave-uniform: a wave past the last key skips the pass
+    bool live = key0 < L;  // wave-uniform: a wave past the last key skips the pass
+    if (one_chain) {
+      bool hit = false;
+#pragma unroll
+      for (int i = 0; i < KW / 64; i++) {
+        kid[i] = kid_next[i];
+        hit = hit || (key0 + 64 * i + lane < L && kid[i] == qsid0);
+      }
+      live = live && __any(hit);
+      key_ids(base + LP, kid_next);
+    }
     // the previous pass's LDS reads have all returned before its MFMAs ran; keep the
     // compiler from moving them past the loads that overwrite the rows
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
@@ -508,10 +531,7 @@ hipError_t launch_esmc_qk_rope(const EsmcRopeArgs& a, hipStream_t s) {
 
 hipError_t launch_esmc_attention(const EsmcAttnArgs& a, hipStream_t s) {
   const dim3 grid(((a.L + 31) / 32) * a.B * a.H);
-  if (a.L <= 256)  // one pass of 256 keys; longer sequences take passes of 512
-    ESM_LAUNCH(esmc_attention_kernel<8>, grid, dim3(256), 0, s, a);
-  else
-    ESM_LAUNCH(esmc_attention_kernel<16>, grid, dim3(256), 0, s, a);
+  ESM_LAUNCH(esmc_attention_kernel, grid, dim3(256), 0, s, a);
   return hipGetLastError();
 }
 

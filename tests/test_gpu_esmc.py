@@ -62,7 +62,7 @@ def test_qk_rope(gpu_lib, pkg, B, L, H):
 @pytest.mark.parametrize("L", [1, 5, 31, 64, 130, 238, 300, 512, 513, 700, 1100])
 @pytest.mark.parametrize("masked", [False, True])
 def test_attention(gpu_lib, pkg, L, masked):
-    # beyond 512 tokens the keys go in passes of 512 with an online softmax: the chains then
+    # beyond 256 tokens the keys go in passes of 256 with an online softmax: the chains then
     # span pass boundaries, and queries of the later chain see no key in the first pass
     B, H = 2, 3
     g = _gen(L + masked)
@@ -96,6 +96,26 @@ def test_attention_keys_only_in_a_later_pass(gpu_lib, pkg):
     assert err <= 1e-2 * float(ref.pow(2).mean().sqrt()), err
     # the lone token's output is its own value row
     assert torch.allclose(o[0, L - 1].view(H, 64).float().cpu(), v[0, :, L - 1].float(), atol=1e-3)
+
+
+@pytest.mark.parametrize("L,lengths", [(257, (100, 157)), (700, (64, 200, 436)), (900, (320, 320, 260)), (520, None)])
+def test_attention_passes_of_other_chains(gpu_lib, pkg, L, lengths):
+    # blocks of queries inside one chain skip the passes that hold other chains' keys only: chains that end on
+    # and off the 64-key and 256-key edges, one that takes up again later, and ids that alternate (no block of
+    # one chain, nothing skipped)
+    B, H = 2, 2
+    g = _gen(L)
+    q, k, v = (2 * torch.randn(B, H, L, 64, generator=g).half() for _ in range(3))
+    if lengths is None:
+        sid = (torch.arange(L) % 3).int().expand(B, L).clone()
+    else:
+        sid = torch.repeat_interleave(torch.arange(len(lengths)), torch.tensor(lengths)).int().expand(B, L).clone()
+        sid[1, L - 40:] = 0  # chain 0 again, after the others
+    o = pkg.kernels.esmc_attention(q.to(DEV), k.to(DEV), v.to(DEV), sid.to(DEV))
+    ref = oe.attention(q.double(), k.double(), v.double(), oe.chain_mask(sid), 0.125)
+    ref = ref.transpose(1, 2).reshape(B, L, H * 64)
+    err = float((o.double().cpu() - ref).abs().max())
+    assert err <= 1e-2 * float(ref.pow(2).mean().sqrt()), err
 
 
 def test_swiglu(gpu_lib, pkg):
