@@ -16,6 +16,10 @@ namespace esm {
 // holding the 8-channel chunks l + 16 t, fp32 statistics) into LDS as fp16, one barrier,
 // D[co][cell] = B[co][:] . LN(u)[cell][:] (fp32 accumulation), then a[co] * z + D in fp32,
 // 16-byte stores (4 consecutive channels per lane and quad).
+// Bound by its four fp32 streams (232 MB at L=238, C=256). All loads of the next tile, z's too, are in flight
+// while a tile computes (96 registers per set at C = 256); with z loaded behind the products and u at the top
+// of its own tile, on inputs the cache does not hold: 58 -> 52 us at L=238 (4.5 TB/s), 224 -> 196 us at L=512;
+// C=128 25.8 -> 26.2 and 104 -> 98 us.
 template <int CC>
 __global__ __launch_bounds__(256, 1) void parcae_step_kernel(ParcaeArgs p) {
   constexpr int OB = CC / 128;       // 32-channel output blocks per wave
@@ -49,25 +53,47 @@ __global__ __launch_bounds__(256, 1) void parcae_step_kernel(ParcaeArgs p) {
 
   const rsrc_t rz = make_rsrc(p.z), ri = make_rsrc(p.z_init), rr = make_rsrc(p.refined), ro = make_rsrc(p.z_out);
   const size_t ncells = p.ncells;
-  for (int tile = blockIdx.x; tile < p.ntiles; tile += gridDim.x) {
-    const size_t cell0 = (size_t)tile * 32;
+  // A tile's loads: the z_init and refined pieces this lane normalises and the z pieces it updates. A tile (or
+  // cell) past the end loads nothing.
+  struct Loads {
+    f32x4 a[2][NCH][2], b[2][NCH][2], z[OB][4];
+  };
+  auto ld4 = [](rsrc_t r, uint32_t off) { return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0)); };
+  auto out_off = [&](int tile, int ob, int r4) -> uint32_t {
+    const size_t cell = (size_t)tile * 32 + r;
+    return cell < ncells ? (uint32_t)((cell * CC + wave * (CC / 4) + 32 * ob + acc_row32(4 * r4, lane)) * 4u) : kOOB;
+  };
+  auto load = [&](Loads& ld, int tile) {
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const size_t cell = (size_t)tile * 32 + (tid >> 4) + 16 * i;
+      const bool live = tile < p.ntiles && cell < ncells;
+#pragma unroll
+      for (int t = 0; t < NCH; t++)
+#pragma unroll
+        for (int hh = 0; hh < 2; hh++) {
+          const uint32_t off = live ? (uint32_t)((cell * CC + 8 * (l16 + 16 * t)) * 4u) + 16u * hh : kOOB;
+          ld.a[i][t][hh] = ld4(ri, off);
+          ld.b[i][t][hh] = ld4(rr, off);
+        }
+    }
+#pragma unroll
+    for (int ob = 0; ob < OB; ob++)
+#pragma unroll
+      for (int r4 = 0; r4 < 4; r4++) ld.z[ob][r4] = ld4(rz, tile < p.ntiles ? out_off(tile, ob, r4) : kOOB);
+  };
+  auto process = [&](const Loads& ld, int tile) {
     // 1. u -> LayerNorm -> LDS
 #pragma unroll
     for (int i = 0; i < 2; i++) {
       const int cl = (tid >> 4) + 16 * i;
-      const bool live = cell0 + cl < ncells;
       float v[NCH][8];
 #pragma unroll
-      for (int t = 0; t < NCH; t++) {
-        const uint32_t off = live ? (uint32_t)(((cell0 + cl) * CC + 8 * (l16 + 16 * t)) * 4u) : kOOB;
+      for (int t = 0; t < NCH; t++)
 #pragma unroll
-        for (int hh = 0; hh < 2; hh++) {
-          const f32x4 a4 = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(ri, (int)(off + 16u * hh), 0, 0));
-          const f32x4 b4 = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rr, (int)(off + 16u * hh), 0, 0));
+        for (int hh = 0; hh < 2; hh++)
 #pragma unroll
-          for (int e = 0; e < 4; e++) v[t][4 * hh + e] = a4[e] + b4[e];
-        }
-      }
+          for (int e = 0; e < 4; e++) v[t][4 * hh + e] = ld.a[i][t][hh][e] + ld.b[i][t][hh][e];
       float s = 0.f;
 #pragma unroll
       for (int t = 0; t < NCH; t++)
@@ -105,20 +131,32 @@ __global__ __launch_bounds__(256, 1) void parcae_step_kernel(ParcaeArgs p) {
       for (int ob = 0; ob < OB; ob++) d[ob] = mfma32(bw[ob][ks], nb, d[ob]);
     }
     // 3. a * z + D for the lane's cell and 4 quads of 4 consecutive channels per block
-    const bool live = cell0 + r < ncells;
 #pragma unroll
     for (int ob = 0; ob < OB; ob++)
 #pragma unroll
       for (int r4 = 0; r4 < 4; r4++) {
-        const int co = wave * (CC / 4) + 32 * ob + acc_row32(4 * r4, lane);
-        const uint32_t off = live ? (uint32_t)(((cell0 + r) * CC + co) * 4u) : kOOB;
-        const f32x4 z4 = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rz, (int)off, 0, 0));
         f32x4 o;
 #pragma unroll
-        for (int e = 0; e < 4; e++) o[e] = av[ob][4 * r4 + e] * z4[e] + d[ob][4 * r4 + e];
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), ro, (int)off, 0, 0);
+        for (int e = 0; e < 4; e++) o[e] = av[ob][4 * r4 + e] * ld.z[ob][r4][e] + d[ob][4 * r4 + e];
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), ro, (int)out_off(tile, ob, r4), 0, 0);
       }
     __syncthreads();  // n_s is rewritten by the next tile
+  };
+  // The next tile's loads are in flight while this one computes, in two register sets (no copy waits on a load).
+  const int G = gridDim.x;
+  Loads l0, l1;
+  int tile = blockIdx.x;
+  load(l0, tile);
+  if (p.ntiles <= G) {  // one tile each: nothing to keep in flight
+    process(l0, tile);
+    return;
+  }
+  for (; tile < p.ntiles; tile += 2 * G) {
+    load(l1, tile + G);
+    process(l0, tile);
+    if (tile + G >= p.ntiles) break;
+    load(l0, tile + 2 * G);
+    process(l1, tile + G);
   }
 }
 
