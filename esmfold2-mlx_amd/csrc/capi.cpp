@@ -7,6 +7,7 @@
 #include <atomic>
 #include <cmath>
 #include <cstdarg>
+#include <cstdint>
 #include <cstdio>
 #include <mutex>
 #include <string>
@@ -80,12 +81,13 @@ constexpr int kQ8MaxK = 1 << 20;  // keeps every per-row byte offset far below 2
 constexpr double kQ8StepUs = 0.7, kQ8NarrowStep = 0.9, kQ8PartialBytesPerUs = 4.0e6;
 std::atomic<int> g_q8_tile_rows{0};  // q8_set_tile_rows: 0 lets the plan choose
 struct Q8Plan {
-  int mtiles, ntiles, splits, nb;
+  int mtiles, ntiles, splits, nb, big;
   size_t bytes;
 };
 Q8Plan q8_plan_nb(int M, int K, int N, int nb) {
   Q8Plan p;
   p.nb = nb;
+  p.big = 0;
   p.mtiles = (M + esm::kQ8TileM - 1) / esm::kQ8TileM;
   p.ntiles = (N + 32 * nb - 1) / (32 * nb);
   const long long tiles = (long long)p.mtiles * p.ntiles;
@@ -104,12 +106,56 @@ double q8_plan_cost(const Q8Plan& p, int M, int K, int N) {
   if (p.splits > 1) c += p.splits * (double)M * N * 8.0 / kQ8PartialBytesPerUs;
   return c;
 }
-Q8Plan q8_plan(int M, int K, int N, bool swiglu = false) {
+// The many-rows form: tiles of 256 rows of x by 160 weight rows, its split count the cheapest by the same kind
+// of estimate: a group of 64 k takes ~1.1 us, a workgroup's start and end ~5.5 (the 64-row form's ~6 per round);
+// up to two workgroups per CU where K is split, so that the partials stay under 84 MB on 256 CUs. It is taken
+// where its estimate is lower and the scratch at hand holds its partials, and only where those are no fewer bytes
+// than the 64-row form's, so that no call is taken with less scratch than that form needs. Measured at M = 512,
+// 700, 900 and 1100, 64-row form / this, us: 2560 -> 10240 45 / 50, 64 / 51, 87 / 51, 103 / 96; 2560 -> 7680 35 / 46,
+// 51 / 47, 63 / 49, 80 / 50; 5120 -> 2560 26 / 33, 31 / 38, 37 / 42, 60 / 47; 2560 -> 2560 21 / 30, 19 / 32, 22 / 36,
+// 35 / 37; 10240 -> 2560 42 / 44, 59 / 56, 71 / 66, 112 / 76.
+constexpr double kQ8BigGroupUs = 1.1, kQ8BigFixedUs = 5.5, kQ8FixedUs = 6.0;
+Q8Plan q8_plan_big(int M, int K, int N, double* cost) {
+  Q8Plan p{};
+  p.nb = esm::kQ8TileNbWide;
+  p.big = 1;
+  p.mtiles = (M + esm::kQ8BigM - 1) / esm::kQ8BigM;
+  p.ntiles = (N + 32 * p.nb - 1) / (32 * p.nb);
+  const long long cus = cu_count(), tiles = (long long)p.mtiles * p.ntiles;
+  const int steps = (K / 64 + 1) / 2;
+  *cost = 1e30;
+  for (int sp = 1; sp == 1 || (sp <= kQ8MaxSplits && 4 * sp <= steps && tiles * sp <= 2 * cus); sp++) {
+    const long long rounds = (tiles * sp + cus - 1) / cus;
+    double c = (double)rounds * (2.0 * ((steps + sp - 1) / sp) * kQ8BigGroupUs + kQ8BigFixedUs);
+    if (sp > 1) c += sp * (double)M * N * 8.0 / kQ8PartialBytesPerUs;
+    if (c < *cost) {
+      *cost = c;
+      p.splits = sp;
+    }
+  }
+  p.bytes = (size_t)p.splits * M * N * sizeof(float);
+  return p;
+}
+Q8Plan q8_plan(int M, int K, int N, bool swiglu = false, size_t scratch = SIZE_MAX) {
   const int forced = g_q8_tile_rows.load() / 32;
-  if (swiglu) return q8_plan_nb(M, K, N, esm::kQ8TileNbWide);
-  if (forced) return q8_plan_nb(M, K, N, forced);
+  if (forced) return q8_plan_nb(M, K, N, swiglu ? esm::kQ8TileNbWide : forced);
   const Q8Plan narrow = q8_plan_nb(M, K, N, esm::kQ8TileNbNarrow), wide = q8_plan_nb(M, K, N, esm::kQ8TileNbWide);
-  return q8_plan_cost(narrow, M, K, N) <= q8_plan_cost(wide, M, K, N) ? narrow : wide;
+  const double cn = q8_plan_cost(narrow, M, K, N), cw = q8_plan_cost(wide, M, K, N);
+  const Q8Plan& small = swiglu || cn > cw ? wide : narrow;
+  // the choice of the form is the same for the plain and the SwiGLU product of a shape, so that both have the
+  // same bits
+  const Q8Plan& best = cn <= cw ? narrow : wide;
+  const long long wgs = (long long)best.mtiles * best.ntiles * best.splits, cus = cu_count();
+  if (wgs > 0x7fffffffLL) return small;
+  double cb;
+  const Q8Plan big = q8_plan_big(M, K, N, &cb);
+  if (cb >= 0.98 * (std::min(cn, cw) + kQ8FixedUs * (double)((wgs + cus - 1) / cus))) return small;
+  const auto need = [](const Q8Plan& p) { return p.splits > 1 ? p.bytes : 0; };
+  return std::max(need(narrow), need(wide)) <= need(big) && need(big) <= scratch ? big : small;
+}
+// The bytes of a caller's workspace that a plan may count on: none where it could not be used.
+size_t q8_usable(const void* ws, size_t bytes) {
+  return ws && (reinterpret_cast<uintptr_t>(ws) & 255u) == 0 ? bytes : 0;
 }
 
 #ifndef ESM_SOURCE_HASH
@@ -550,7 +596,7 @@ int q8_linear_ws(const esm_half* x, const uint8_t* q, const esm_half* s, const e
   bool empty;
   if (const int rc = q8_check("q8_linear", x, q, s, b, y, 8, M, K, N, group, &empty)) return rc;
   if (empty) return ok();
-  Q8Plan pl = q8_plan(M, K, N);
+  Q8Plan pl = q8_plan(M, K, N, false, q8_usable(workspace, workspace_bytes));
   if ((long long)pl.mtiles * pl.ntiles * pl.splits > 0x7fffffffLL)
     return fail(ESM_ERR_SHAPE, "q8_linear: M=%d N=%d too large", M, N);
   if (!workspace) {
@@ -563,7 +609,7 @@ int q8_linear_ws(const esm_half* x, const uint8_t* q, const esm_half* s, const e
   }
   if (sb && !aligned16(sb)) return fail(ESM_ERR_ALIGN, "q8_linear: packed scales must be 16-byte aligned");
   esm::Q8Args a{H(x), q, H(s), H(b), H(y), M, K, N, pl.mtiles, pl.ntiles, pl.splits,
-                pl.splits > 1 ? static_cast<float*>(workspace) : nullptr, sb, nullptr, 0, pl.nb};
+                pl.splits > 1 ? static_cast<float*>(workspace) : nullptr, sb, nullptr, 0, pl.nb, pl.big};
   return hip_status(esm::launch_q8_linear(a, (hipStream_t)stream), "q8_linear launch");
 }
 
@@ -573,7 +619,7 @@ int q8_linear_noalloc(const esm_half* x, const uint8_t* q, const esm_half* s, co
   bool empty;
   if (const int rc = q8_check("q8_linear_noalloc", x, q, s, b, y, 8, M, K, N, group, &empty)) return rc;
   if (empty) return ok();
-  const Q8Plan pl = q8_plan(M, K, N);
+  const Q8Plan pl = q8_plan(M, K, N, false, esm::kQ8ScratchBytes);
   if ((long long)pl.mtiles * pl.ntiles * pl.splits > 0x7fffffffLL)
     return fail(ESM_ERR_SHAPE, "q8_linear_noalloc: M=%d N=%d too large", M, N);
   if (pl.splits > 1 && pl.bytes > esm::kQ8ScratchBytes)
@@ -585,7 +631,8 @@ int q8_linear_noalloc(const esm_half* x, const uint8_t* q, const esm_half* s, co
     const hipError_t e = esm::q8_scratch_address(&part);
     if (e != hipSuccess) return hip_status(e, "q8_linear_noalloc: scratch address");
   }
-  esm::Q8Args a{H(x), q, H(s), H(b), H(y), M, K, N, pl.mtiles, pl.ntiles, pl.splits, part, sb, nullptr, 0, pl.nb};
+  esm::Q8Args a{H(x), q, H(s), H(b), H(y), M, K, N, pl.mtiles, pl.ntiles, pl.splits, part,
+                sb, nullptr, 0, pl.nb, pl.big};
   return hip_status(esm::launch_q8_linear(a, (hipStream_t)stream), "q8_linear_noalloc launch");
 }
 
@@ -601,14 +648,15 @@ int q8_linear_partials(const esm_half* x, const uint8_t* q, const esm_half* s, c
   *splits = 0;
   if (const int rc = q8_check("q8_linear_partials", x, q, s, b, parts, 256, M, K, N, group, &empty)) return rc;
   if (empty) return ok();
-  const Q8Plan pl = q8_plan(M, K, N);
+  const Q8Plan pl = q8_plan(M, K, N, false, parts_bytes);
   if ((long long)pl.mtiles * pl.ntiles * pl.splits > 0x7fffffffLL)
     return fail(ESM_ERR_SHAPE, "q8_linear_partials: M=%d N=%d too large", M, N);
   if (parts_bytes < pl.bytes)
     return fail(ESM_ERR_SHAPE, "q8_linear_partials: %zu bytes for the partials, %zu needed", parts_bytes, pl.bytes);
   if (sb && !aligned16(sb)) return fail(ESM_ERR_ALIGN, "q8_linear_partials: packed scales must be 16-byte aligned");
   *splits = pl.splits;
-  esm::Q8Args a{H(x), q, H(s), H(b), nullptr, M, K, N, pl.mtiles, pl.ntiles, pl.splits, parts, sb, nullptr, 0, pl.nb};
+  esm::Q8Args a{H(x), q, H(s), H(b), nullptr, M, K, N, pl.mtiles, pl.ntiles, pl.splits, parts,
+                sb, nullptr, 0, pl.nb, pl.big};
   return hip_status(esm::launch_q8_linear(a, (hipStream_t)stream), "q8_linear_partials launch");
 }
 
@@ -620,7 +668,7 @@ int q8_linear_packed_ws(const esm_half* x, const uint8_t* qp, const uint32_t* sb
                                       &empty))
     return rc;
   if (empty) return ok();
-  Q8Plan pl = q8_plan(M, K, N);
+  Q8Plan pl = q8_plan(M, K, N, false, q8_usable(workspace, workspace_bytes));
   if ((long long)pl.mtiles * pl.ntiles * pl.splits > 0x7fffffffLL)
     return fail(ESM_ERR_SHAPE, "q8_linear_packed_ws: M=%d N=%d too large", M, N);
   if (!workspace) {
@@ -632,7 +680,7 @@ int q8_linear_packed_ws(const esm_half* x, const uint8_t* qp, const uint32_t* sb
       return fail(ESM_ERR_ALIGN, "q8_linear_packed_ws: workspace must be 256-byte aligned");
   }
   esm::Q8Args a{H(x), nullptr, nullptr, nullptr, H(y), M, K, N, pl.mtiles, pl.ntiles, pl.splits,
-                pl.splits > 1 ? static_cast<float*>(workspace) : nullptr, sb, qp, 0, pl.nb};
+                pl.splits > 1 ? static_cast<float*>(workspace) : nullptr, sb, qp, 0, pl.nb, pl.big};
   return hip_status(esm::launch_q8_linear(a, (hipStream_t)stream), "q8_linear_packed_ws launch");
 }
 
@@ -647,7 +695,7 @@ int q8_linear_swiglu_packed_ws(const esm_half* x, const uint8_t* qp, const uint3
   if (N % (2 * esm::kQ8SwigluHalf) != 0)
     return fail(ESM_ERR_SHAPE, "q8_linear_swiglu_packed_ws: N=%d must be a multiple of %d (SwiGLU pair tiles)", N,
                 2 * esm::kQ8SwigluHalf);
-  Q8Plan pl = q8_plan(M, K, N, true);
+  Q8Plan pl = q8_plan(M, K, N, true, q8_usable(workspace, workspace_bytes));
   if ((long long)pl.mtiles * pl.ntiles * pl.splits > 0x7fffffffLL)
     return fail(ESM_ERR_SHAPE, "q8_linear_swiglu_packed_ws: M=%d N=%d too large", M, N);
   if (!workspace) {
@@ -660,7 +708,7 @@ int q8_linear_swiglu_packed_ws(const esm_half* x, const uint8_t* qp, const uint3
       return fail(ESM_ERR_ALIGN, "q8_linear_swiglu_packed_ws: workspace must be 256-byte aligned");
   }
   esm::Q8Args a{H(x), nullptr, nullptr, nullptr, H(y), M, K, N, pl.mtiles, pl.ntiles, pl.splits,
-                pl.splits > 1 ? static_cast<float*>(workspace) : nullptr, sb, qp, 1, pl.nb};
+                pl.splits > 1 ? static_cast<float*>(workspace) : nullptr, sb, qp, 1, pl.nb, pl.big};
   return hip_status(esm::launch_q8_linear(a, (hipStream_t)stream), "q8_linear_swiglu_packed_ws launch");
 }
 
@@ -674,14 +722,15 @@ int q8_linear_packed_partials(const esm_half* x, const uint8_t* qp, const uint32
                                       K, N, group, &empty))
     return rc;
   if (empty) return ok();
-  const Q8Plan pl = q8_plan(M, K, N);
+  const Q8Plan pl = q8_plan(M, K, N, false, parts_bytes);
   if ((long long)pl.mtiles * pl.ntiles * pl.splits > 0x7fffffffLL)
     return fail(ESM_ERR_SHAPE, "q8_linear_packed_partials: M=%d N=%d too large", M, N);
   if (parts_bytes < pl.bytes)
     return fail(ESM_ERR_SHAPE, "q8_linear_packed_partials: %zu bytes for the partials, %zu needed", parts_bytes,
                 pl.bytes);
   *splits = pl.splits;
-  esm::Q8Args a{H(x), nullptr, nullptr, nullptr, nullptr, M, K, N, pl.mtiles, pl.ntiles, pl.splits, parts, sb, qp, 0, pl.nb};
+  esm::Q8Args a{H(x), nullptr, nullptr, nullptr, nullptr, M, K, N, pl.mtiles, pl.ntiles, pl.splits, parts,
+                sb, qp, 0, pl.nb, pl.big};
   return hip_status(esm::launch_q8_linear(a, (hipStream_t)stream), "q8_linear_packed_partials launch");
 }
 

@@ -80,11 +80,13 @@ struct Q8Args {
   int swiglu;           // weight rows in SwiGLU pairs (each 160-row tile: 80 gate rows, then the
                         // matching 80 up rows): y [M, N/2] = silu(gate) * up instead of [M, N]
   int nb;               // 32-row weight blocks per tile: kQ8TileNbNarrow or kQ8TileNbWide
+  int big;              // tiles of kQ8BigM rows of x x 160 weight rows (mtiles counts those)
 };
 
 // q8 GEMM tile: kQ8TileM rows of x by 32 nb weight rows (nb = 4 or 5, chosen per call by the
 // launch plan), kQ8Waves waves per workgroup. The packed layouts do not depend on nb.
 constexpr int kQ8TileM = 64;
+constexpr int kQ8BigM = 256;  // rows of x per tile of the many-rows form
 constexpr int kQ8TileNbNarrow = 4;
 constexpr int kQ8TileNbWide = 5;
 constexpr int kQ8Waves = 4;

@@ -423,6 +423,204 @@ __global__ __launch_bounds__(NWQ * 64, 1) void q8_linear_kernel(Q8Args p) {
   }
 }
 
+// ---- the same product on 256 x 160 tiles, for many rows of x ------------------------------------
+// With x longer than a few tiles of 64 rows the kernel above dequantises every weight once per 64 rows, on one
+// wave per SIMD. Here an 8-wave workgroup owns 256 rows of x and 160 weight rows; each group of 64 k is
+// dequantised once, a share per wave, into LDS (fp16, the same values), and every wave multiplies its 64 x 80
+// outputs (4 x 5 of v_mfma_f32_16x16x32_f16) from there. x comes by loads that write LDS, a ring of three
+// groups; the codes of a 128-k step wait in registers, two steps ahead. One barrier per group. A group takes
+// ~1.1 us (2,300 cycles against 1,280 of MFMAs on a SIMD): the dequantisation and the requests of all waves
+// precede their products. M = 1100: 2560 -> 7680 80 -> 50 us (0.86 PFLOP/s), 2560 -> 10240 103 -> 96, 5120 -> 2560
+// 60 -> 47, 10240 -> 2560 112 -> 76.
+namespace {
+constexpr int BGM = kQ8BigM, BGN = 32 * kQ8TileNbWide, BGT = 512;
+constexpr int BXS = BGM * 128, BWS = BGN * 128;      // bytes of a group of x and of dequantised weights
+constexpr int BCH = (kQ8TileNbWide * 4 + 7) / 8;     // 1 KB code chunks per wave and step (the last on waves 0-3 only)
+constexpr int BSTR = BGN + 8;                        // output staging row stride (halfs)
+}  // namespace
+
+template <bool PC, bool PSB>  // codes, scales in their packed layouts
+__global__ __launch_bounds__(BGT, 1) void q8_linear_big_kernel(Q8Args p) {
+  constexpr int SMEM = 3 * BXS + 2 * BWS;
+  static_assert(BGM * BSTR * 2 <= SMEM && SMEM <= 160 * 1024, "LDS");
+  __shared__ __align__(1024) char smem[SMEM];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1, l16 = lane & 15, q4 = lane >> 4;
+  // the m-tiles of one n-tile are neighbours in the XCD-aware order and read its codes from one L2
+  int t = xcd_remap(blockIdx.x, gridDim.x);
+  const int mt = t % p.mtiles;
+  t /= p.mtiles;
+  const int nt = t % p.ntiles, sp = t / p.ntiles;
+  const int m0 = mt * BGM, n0 = nt * BGN, blk0 = n0 / 32;
+  const int K = p.K, M = p.M, N = p.N, ngroups = K / QG, S = (ngroups + 1) / 2;
+  const int st0 = (int)((long long)S * sp / p.splits), st1 = (int)((long long)S * (sp + 1) / p.splits);
+  const int sg0 = 2 * st0, n = (2 * st1 < ngroups ? 2 * st1 : ngroups) - sg0, nst = st1 - st0;
+  const int nblk = (N + 31) / 32 - blk0 < kQ8TileNbWide ? (N + 31) / 32 - blk0 : kQ8TileNbWide;
+  const uint32_t lds0 = lds_address(smem);
+
+  // --- x: 8 rows of 128 bytes per load, 16-byte pieces XOR-swizzled by the row
+  const uint64_t xbytes = (uint64_t)(M - m0) * (uint64_t)K * 2u;
+  const dma_src_t rx = dma_src(p.x + (size_t)m0 * K, (uint32_t)(xbytes < 0x7ffffff0ull ? xbytes : 0x7ffffff0ull));
+  auto load_x = [&](int s) {  // group sg0 + s
+    const uint32_t dst = lds0 + (s % 3) * BXS + wave * 4096;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int row = 32 * wave + 8 * i + (lane >> 3);
+      const uint32_t off = (uint32_t)row * (uint32_t)K * 2u + 16u * ((lane & 7) ^ ((row >> 1) & 7));
+      dma16(rx, dst + i * 1024, s < n ? off + (uint32_t)(sg0 + s) * 128u : kOOB, 0);
+    }
+  };
+  // --- codes of a step (two groups) and their scales: chunk c of this wave is block nb, k 16 kk .. + 15 of both
+  const rsrc_t rq = PC ? make_rsrc_n(p.qp + (size_t)blk0 * S * 4096u, (uint32_t)nblk * (uint32_t)S * 4096u)
+                       : make_rsrc_n(p.q + (size_t)n0 * K, (uint32_t)(N - n0) * (uint32_t)K);
+  const rsrc_t rs = PSB ? make_rsrc_n(p.sb + (size_t)blk0 * ngroups * 32, (uint32_t)nblk * (uint32_t)ngroups * 128u)
+                        : make_rsrc_n(p.s + (size_t)n0 * ngroups, (uint32_t)(N - n0) * (uint32_t)ngroups * 2u);
+  const rsrc_t rb = PSB ? rs : make_rsrc_n(p.b + (size_t)n0 * ngroups, (uint32_t)(N - n0) * (uint32_t)ngroups * 2u);
+  struct Codes {
+    u32x4 q[BCH];
+    uint32_t sb[BCH][2];
+  };
+  auto load_codes = [&](Codes& c, int j) {  // step st0 + j
+    const bool live = j < nst;
+    const int st = st0 + j;
+#pragma unroll
+    for (int i = 0; i < BCH; i++) {
+      const int id = wave + 8 * i, nb = id >> 2, kk = id & 3, row = 32 * nb + (lane & 31);
+      const bool ok = live && id < 4 * kQ8TileNbWide, two = 2 * st + 1 < ngroups;
+      if constexpr (PC) {
+        c.q[i] = __builtin_amdgcn_raw_buffer_load_b128(
+            rq, (int)(ok ? ((uint32_t)nb * S + st) * 4096u + kk * 1024u + lane * 16u : kOOB), 0, 0);
+      } else {
+        const uint32_t off = (uint32_t)row * K + 128u * st + 16u * kk + 8u * (lane >> 5);
+        const u32x2 lo = __builtin_amdgcn_raw_buffer_load_b64(rq, (int)(ok ? off : kOOB), 0, 0);
+        const u32x2 hi = __builtin_amdgcn_raw_buffer_load_b64(rq, (int)(ok && two ? off + 64u : kOOB), 0, 0);
+        c.q[i] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+      }
+#pragma unroll
+      for (int g = 0; g < 2; g++) {
+        const bool okg = ok && (g == 0 || two);
+        if constexpr (PSB) {
+          const uint32_t off = (((uint32_t)nb * ngroups + 2 * st + g) * 32u + (lane & 31)) * 4u;
+          c.sb[i][g] = __builtin_amdgcn_raw_buffer_load_b32(rs, (int)(okg ? off : kOOB), 0, 0);
+        } else {
+          const uint32_t off = ((uint32_t)row * ngroups + 2 * st + g) * 2u;
+          c.sb[i][g] = (uint32_t)bload2(rb, okg ? off : kOOB) << 16 | bload2(rs, okg ? off : kOOB);
+        }
+      }
+    }
+  };
+  auto dequant = [&](const Codes& c, int g, int buf) {
+#pragma unroll
+    for (int i = 0; i < BCH; i++) {
+      const int id = wave + 8 * i, row = 32 * (id >> 2) + (lane & 31), piece = 2 * (id & 3) + (lane >> 5);
+      if (id < 4 * kQ8TileNbWide)
+        *reinterpret_cast<half8*>(smem + 3 * BXS + buf * BWS + row * 128 + 16 * (piece ^ ((row >> 1) & 7))) =
+            dequant8(c.q[i][2 * g], c.q[i][2 * g + 1], splat2(c.sb[i][g] & 0xffffu), splat2(c.sb[i][g] >> 16));
+    }
+  };
+  f32x4 acc[4][5];
+#pragma unroll
+  for (int mi = 0; mi < 4; mi++)
+#pragma unroll
+    for (int ni = 0; ni < 5; ni++) acc[mi][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto products = [&](int s) {
+    const int sw = (l16 >> 1) & 7;  // every row here is l16 plus a multiple of 16
+    const char* xs = smem + (s % 3) * BXS + (64 * wm + l16) * 128;
+    const char* ws = smem + 3 * BXS + (s & 1) * BWS + (80 * wn + l16) * 128;
+#pragma unroll
+    for (int ks = 0; ks < 2; ks++) {
+      const int at = 16 * ((4 * ks + q4) ^ sw);
+      half8 xf[4], wf[5];
+#pragma unroll
+      for (int mi = 0; mi < 4; mi++) xf[mi] = *reinterpret_cast<const half8*>(xs + mi * 2048 + at);
+#pragma unroll
+      for (int ni = 0; ni < 5; ni++) wf[ni] = *reinterpret_cast<const half8*>(ws + ni * 2048 + at);
+#pragma unroll
+      for (int ni = 0; ni < 5; ni++)
+#pragma unroll
+        for (int mi = 0; mi < 4; mi++) acc[mi][ni] = mfma16(wf[ni], xf[mi], acc[mi][ni]);  // D[n][m]
+    }
+  };
+  // Group s: the weights of group s + 1 are dequantised (half g of a step's codes) and x of group s + 2 is
+  // requested before the products (requesting x first and leaving the order of the rest to the compiler took
+  // 57 us where this takes 50); what is loaded beyond the range is zero and adds nothing.
+  auto group = [&](int s, Codes& c, int g, int reload) {
+    dequant(c, g, (s + 1) & 1);
+    if (reload >= 0) load_codes(c, reload);
+    load_x(s + 2);
+    products(s);
+    wait_vm(4);  // x of group s + 1 is in LDS; only group s + 2's loads came after every other load
+    __syncthreads();
+  };
+  Codes ca, cb;
+  load_codes(ca, 0);
+  load_x(0);
+  load_x(1);
+  load_codes(cb, 1);
+  dequant(ca, 0, 0);
+  wait_vm(0);
+  __syncthreads();
+  for (int j = 0; j < nst; j += 2) {
+    group(2 * j, ca, 1, j + 2);
+    group(2 * j + 1, cb, 0, -1);
+    if (j + 1 < nst) {
+      group(2 * j + 2, cb, 1, j + 3);
+      group(2 * j + 3, ca, 0, -1);
+    }
+  }
+  wait_vm(0);
+  __syncthreads();
+
+  if (p.part) {  // fp32 partials (summed by the reduction or the consumer)
+    float* part = p.part + (size_t)sp * M * N;
+#pragma unroll
+    for (int mi = 0; mi < 4; mi++)
+#pragma unroll
+      for (int ni = 0; ni < 5; ni++) {
+        const int m = m0 + 64 * wm + 16 * mi + l16, nn = n0 + 80 * wn + 16 * ni + 4 * q4;
+        if (m < M && nn < N) *reinterpret_cast<f32x4*>(part + (size_t)m * N + nn) = acc[mi][ni];
+      }
+    return;
+  }
+  half_t* os = reinterpret_cast<half_t*>(smem);
+#pragma unroll
+  for (int mi = 0; mi < 4; mi++)
+#pragma unroll
+    for (int ni = 0; ni < 5; ni++)
+      *reinterpret_cast<half4*>(os + (64 * wm + 16 * mi + l16) * BSTR + 80 * wn + 16 * ni + 4 * q4) =
+          half4{(half_t)acc[mi][ni][0], (half_t)acc[mi][ni][1], (half_t)acc[mi][ni][2], (half_t)acc[mi][ni][3]};
+  __syncthreads();
+  if (p.swiglu) {  // 80 gate rows, then their up rows: both rounded to fp16 as y would be, as esmc_swiglu does
+    const int F = N / 2;
+    for (int id = tid; id < BGM * (kQ8SwigluHalf / 8); id += BGT) {
+      const int row = id / (kQ8SwigluHalf / 8), pcs = id - row * (kQ8SwigluHalf / 8);
+      const half8 g = ld16(os + row * BSTR + 8 * pcs), u = ld16(os + row * BSTR + kQ8SwigluHalf + 8 * pcs);
+      half8 o;
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const float v = (float)g[e];
+        o[e] = (half_t)(v * sigmoidf_fast(v) * (float)u[e]);
+      }
+      if (m0 + row < M) {
+        half_t* d = p.y + (size_t)(m0 + row) * F + nt * kQ8SwigluHalf + 8 * pcs;  // 8-byte aligned
+        *reinterpret_cast<half4*>(d) = half4{o[0], o[1], o[2], o[3]};
+        *reinterpret_cast<half4*>(d + 4) = half4{o[4], o[5], o[6], o[7]};
+      }
+    }
+    return;
+  }
+  for (int id = tid; id < BGM * (BGN / 8); id += BGT) {
+    const int row = id / (BGN / 8), pcs = id - row * (BGN / 8);
+    if (m0 + row < M && n0 + 8 * pcs < N) {
+      half_t* d = p.y + (size_t)(m0 + row) * N + n0 + 8 * pcs;  // 8-byte aligned
+      const half8 v = ld16(os + row * BSTR + 8 * pcs);
+      *reinterpret_cast<half4*>(d) = half4{v[0], v[1], v[2], v[3]};
+      *reinterpret_cast<half4*>(d + 4) = half4{v[4], v[5], v[6], v[7]};
+    }
+  }
+}
+
 // y = sum of the split partials in split order (deterministic), one rounding to fp16.
 // Four outputs per thread; M * N is a multiple of 64.
 __global__ __launch_bounds__(256) void q8_reduce_kernel(const float* __restrict__ part, half_t* __restrict__ y,
@@ -572,7 +770,14 @@ hipError_t launch_q8_linear(const Q8Args& a, hipStream_t s) {
     ESM_LAUNCH((q8_linear_kernel<true, false, NB>), dim3(grid), dim3(NWQ * 64), 0, s, a); \
   else                                                                                 \
     ESM_LAUNCH((q8_linear_kernel<false, false, NB>), dim3(grid), dim3(NWQ * 64), 0, s, a);
-  if (a.nb == kQ8TileNbWide) {
+  if (a.big) {
+    if (a.qp)
+      ESM_LAUNCH((q8_linear_big_kernel<true, true>), dim3(grid), dim3(BGT), 0, s, a);
+    else if (a.sb)
+      ESM_LAUNCH((q8_linear_big_kernel<false, true>), dim3(grid), dim3(BGT), 0, s, a);
+    else
+      ESM_LAUNCH((q8_linear_big_kernel<false, false>), dim3(grid), dim3(BGT), 0, s, a);
+  } else if (a.nb == kQ8TileNbWide) {
     Q8_LAUNCH(kQ8TileNbWide)
   } else {
     Q8_LAUNCH(kQ8TileNbNarrow)

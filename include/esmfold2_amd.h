@@ -275,12 +275,14 @@ int q8_linear(const esm_half* x, const uint8_t* q, const esm_half* s, const esm_
  * weights) can afford:
  *   sb: the scales and biases pre-packed by q8_pack_scales (once per weight matrix);
  *       NULL reads them from s and b (slower: 128-160 scattered rows per 128-wide step).
- *   workspace: for shapes whose output tiles (64 x 128 or 64 x 160, q8_tile_rows) are too
+ *   workspace: for shapes whose output tiles (64 x 128 or 64 x 160, q8_tile_rows, or
+ *       256 x 160 for many rows of x: the launch plan's estimate of the faster one) are too
  *       few to fill the GPU (e.g. M = 238, N = 2560), K is split over several workgroups whose fp32
  *       partials go through the workspace and are summed in split order by a second
  *       kernel on the same stream (deterministic). q8_linear_workspace_bytes(M, K, N)
- *       bytes, 256-byte aligned, no initialisation needed; NULL runs unsplit. Calls
- *       that share a workspace must not overlap in time.
+ *       bytes, 256-byte aligned, no initialisation needed; NULL runs unsplit. A workspace
+ *       that holds only the partials of the 64-row tiles (none where those need none) gets
+ *       the 64-row tiles. Calls that share a workspace must not overlap in time.
  * s and b are required either way. Same semantics and result as q8_linear
  * (mx.quantized_matmul, mlx_esmc.py:78-81); packed or not, the bits are identical.
  */
@@ -297,11 +299,11 @@ size_t q8_linear_workspace_bytes(int M, int K, int N);
  * 128-wide K steps per workgroup x a step's time (a 128-row step ~0.9 of a 160-row one),
  * plus, where K is split, the fp32 partials' write and read (160 always for the SwiGLU-pair
  * call). At M = 238: 128 for N = 7680 and for N = 2560 at K = 2560, 160 for N = 10240 and for
- * N = 2560 at K = 5120 or 10240.
- * Either width gives the same bits when K is not split (it only changes which workgroup
+ * N = 2560 at K = 5120 or 10240. Shapes on 256 x 160 tiles (many rows of x) report 160.
+ * Either width of the 64-row tiles gives the same bits when K is not split (it only changes which workgroup
  * computes an output); with a K split the split count, and so the fp32 summation order,
  * can differ. q8_set_tile_rows(128 or 160) fixes the width for every later plan of this
- * process (0 restores the choice; tests and tuning). No reference counterpart: the
+ * process, on 64-row tiles (0 restores the choice; tests and tuning). No reference counterpart: the
  * reference's quantized_matmul (mlx_esmc.py:78-81) tiles inside MLX.
  */
 int q8_tile_rows(int M, int K, int N);
@@ -464,10 +466,11 @@ int abs_diff_quantile_ws(const float* x, const float* y, size_t n, float q, floa
  * q8_linear_ws without a workspace, for callers that cannot allocate device memory (code
  * under HIP graph capture, serving loops that forbid allocation). No counterpart in the
  * reference: its MLX quantized_matmul allocates its own outputs. Same plan and same bits
- * as q8_linear_ws with a workspace; the split-K partials live in a static device array of
+ * as q8_linear_ws with a workspace of this size; the split-K partials live in a static device array of
  * ESM_Q8_NOALLOC_SCRATCH_BYTES per GPU (taken by the library for the life of the
  * process). A shape whose partials exceed it is refused with ESM_ERR_SHAPE (with 256
- * compute units the plan needs at most about 10.5 MB). Nothing is allocated and nothing
+ * compute units the 64-row tiles need at most about 10.5 MB; where the partials of the
+ * 256-row tiles exceed it the 64-row ones run). Nothing is allocated and nothing
  * needs clearing between calls; calls that overlap in time on one GPU share the array and
  * race, so a caller serialises them (one stream, or its own ordering).
  */

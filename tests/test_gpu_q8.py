@@ -279,6 +279,47 @@ def test_q8_swiglu_fused_same_bits(gpu_lib, pkg, M, K, N):
     assert rel <= 3e-3, f"normwise relative error {rel:.3e}"  # the GEMM's ~3e-4 and two fp16 roundings
 
 
+@pytest.mark.parametrize("M,K,N", [
+    (1100, 2560, 2560 * 3),   # 5 row tiles (the last of 76 rows), unsplit
+    (769, 2560, 2560 * 4),    # a last row tile of one row, SwiGLU pairs in the epilogue
+    (1100, 5120, 2560),       # K split, 33 MB of partials
+    (1024, 4160, 2624),       # an odd number of K groups, a last weight tile of 64 rows, split
+    (2049, 448, 10240),       # 7 groups: fewer steps than the pipeline is deep, unsplit
+])
+def test_q8_many_rows(gpu_lib, pkg, M, K, N):
+    # 256-row tiles (the plan's choice here) against the fp64 product of the same fp16 weights; packed or not and
+    # as partials, the same bits; against the 64-row tiles, which also run where the workspace is too small
+    K_ = pkg.kernels
+    x, q, s, b = (_t(a) for a in q8.make_q8_inputs(M, K, N, seed=M + N))
+    sb, qp = K_.q8_pack_scales(s, b), K_.q8_pack_codes(q)
+    ws = K_.q8_workspace(M, K, N)
+    y = K_.q8_linear(x, q, s, b, workspace=ws)
+    for kw in (dict(packed=sb), dict(packed=sb, codes=qp)):
+        assert torch.equal(K_.q8_linear(x, q, s, b, workspace=ws, **kw).view(torch.int16), y.view(torch.int16))
+    parts, n = K_.q8_linear_partials(x, q, s, b, K_.q8_partials_buffer(M, K, N), packed=sb, codes=qp)
+    total = parts[0].clone()
+    for i in range(1, n):
+        total += parts[i]
+    assert torch.equal(total.half().view(torch.int16), y.view(torch.int16))
+    want = x.double() @ K_.q8_dequant(q, s, b).double().T
+    mag = x.double().abs() @ K_.q8_dequant(q, s, b).double().abs().T
+    # K fp32 sums (K 2^-24 of the sum of magnitudes, at the worst) and one fp16 rounding (2^-11, 2^-25 below the
+    # normal range)
+    bar = mag * K * 2.0 ** -24 + want.abs() * 2.0 ** -11 + 2.0 ** -25
+    assert ((y.double() - want).abs() <= bar).all()
+    with _tile_rows(pkg, 160):
+        y64 = K_.q8_linear(x, q, s, b, workspace=K_.q8_workspace(M, K, N))
+    assert ((y64.double() - want).abs() <= bar).all()
+    assert K_.q8_linear(x, q, s, b).shape == y.shape  # no workspace: unsplit
+    if n > 1:
+        assert ((K_.q8_linear(x, q, s, b, packed=sb, codes=qp).double() - want).abs() <= bar).all()
+    if N % 320 == 0:
+        perm = K_.swiglu_pair_rows(N, DEV)
+        got = K_.q8_linear_swiglu(x, K_.q8_pack_codes(q[perm].contiguous()),
+                                  K_.q8_pack_scales(s[perm].contiguous(), b[perm].contiguous()), N, workspace=ws)
+        assert torch.equal(got.view(torch.int16), K_.esmc_swiglu(y).view(torch.int16))
+
+
 def test_q8_module_swiglu_pairs(gpu_lib, pkg):
     x, q, s, b = (_t(a) for a in q8.make_q8_inputs(238, 640, 1280, seed=9))
     lin = pkg.q8.Q8Linear(q, s, b, device=DEV)
