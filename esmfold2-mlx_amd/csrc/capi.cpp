@@ -82,12 +82,13 @@ constexpr double kQ8StepUs = 0.7, kQ8NarrowStep = 0.9, kQ8PartialBytesPerUs = 4.
 std::atomic<int> g_q8_tile_rows{0};  // q8_set_tile_rows: 0 lets the plan choose
 struct Q8Plan {
   int mtiles, ntiles, splits, nb, big;
+  int head;  // rows on 256-row tiles where the rest runs 64-row ones (0: one form for all)
   size_t bytes;
 };
 Q8Plan q8_plan_nb(int M, int K, int N, int nb) {
   Q8Plan p;
   p.nb = nb;
-  p.big = 0;
+  p.big = p.head = 0;
   p.mtiles = (M + esm::kQ8TileM - 1) / esm::kQ8TileM;
   p.ntiles = (N + 32 * nb - 1) / (32 * nb);
   const long long tiles = (long long)p.mtiles * p.ntiles;
@@ -111,9 +112,9 @@ double q8_plan_cost(const Q8Plan& p, int M, int K, int N) {
 // up to two workgroups per CU where K is split, so that the partials stay under 84 MB on 256 CUs. It is taken
 // where its estimate is lower and the scratch at hand holds its partials, and only where those are no fewer bytes
 // than the 64-row form's, so that no call is taken with less scratch than that form needs. Measured at M = 512,
-// 700, 900 and 1100, 64-row form / this, us: 2560 -> 10240 45 / 50, 64 / 51, 87 / 51, 103 / 96; 2560 -> 7680 35 / 46,
-// 51 / 47, 63 / 49, 80 / 50; 5120 -> 2560 26 / 33, 31 / 38, 37 / 42, 60 / 47; 2560 -> 2560 21 / 30, 19 / 32, 22 / 36,
-// 35 / 37; 10240 -> 2560 42 / 44, 59 / 56, 71 / 66, 112 / 76.
+// 700, 900 and 1100, 64-row form / this, us: 2560 -> 10240 45 / 50, 64 / 51, 87 / 51, 103 / 96 (78 with the row
+// split below); 2560 -> 7680 35 / 46, 51 / 47, 63 / 49, 80 / 50; 5120 -> 2560 26 / 33, 31 / 38, 37 / 42, 60 / 47;
+// 2560 -> 2560 21 / 30, 19 / 32, 22 / 36, 35 / 37; 10240 -> 2560 42 / 44, 59 / 56, 71 / 66, 112 / 76.
 constexpr double kQ8BigGroupUs = 1.1, kQ8BigFixedUs = 5.5, kQ8FixedUs = 6.0;
 Q8Plan q8_plan_big(int M, int K, int N, double* cost) {
   Q8Plan p{};
@@ -131,6 +132,22 @@ Q8Plan q8_plan_big(int M, int K, int N, double* cost) {
     if (c < *cost) {
       *cost = c;
       p.splits = sp;
+    }
+  }
+  // Where the tiles leave a last round mostly empty: whole rounds of them, then the remaining rows on 64-row
+  // tiles in a launch of their own, if the estimate is lower (2560 -> 10240 at M = 1100 107 -> 78 us, at 2200 154 -> 135;
+  // 2560 -> 7680 at M = 1300 91 -> 76, at 1500 110 -> 78).
+  const long long rows = tiles / cus * cus / p.ntiles * esm::kQ8BigM;
+  if (rows > 0 && rows < M) {
+    Q8Plan rest = q8_plan_nb(M - (int)rows, K, N, p.nb);
+    rest.splits = 1;
+    const long long wgs = (long long)rest.mtiles * rest.ntiles, hr = (rows / esm::kQ8BigM * p.ntiles + cus - 1) / cus;
+    const double c = (double)hr * (2.0 * steps * kQ8BigGroupUs + kQ8BigFixedUs) +
+                     q8_plan_cost(rest, (int)(M - rows), K, N) + kQ8FixedUs * (double)((wgs + cus - 1) / cus);
+    if (c < *cost) {
+      *cost = c;
+      p.splits = 1;
+      p.head = (int)rows;
     }
   }
   p.bytes = (size_t)p.splits * M * N * sizeof(float);
@@ -156,6 +173,22 @@ Q8Plan q8_plan(int M, int K, int N, bool swiglu = false, size_t scratch = SIZE_M
 // The bytes of a caller's workspace that a plan may count on: none where it could not be used.
 size_t q8_usable(const void* ws, size_t bytes) {
   return ws && (reinterpret_cast<uintptr_t>(ws) & 255u) == 0 ? bytes : 0;
+}
+
+hipError_t q8_launch(const esm::Q8Args& all, const Q8Plan& pl, hipStream_t st) {
+  if (!pl.head) return esm::launch_q8_linear(all, st);
+  esm::Q8Args a = all;
+  a.M = pl.head;
+  a.mtiles = pl.head / esm::kQ8BigM;
+  if (const hipError_t e = esm::launch_q8_linear(a, st); e != hipSuccess) return e;
+  a = all;
+  a.big = 0;
+  a.M = all.M - pl.head;
+  a.mtiles = (a.M + esm::kQ8TileM - 1) / esm::kQ8TileM;
+  a.x += (size_t)pl.head * a.K;
+  if (a.y) a.y += (size_t)pl.head * (a.swiglu ? a.N / 2 : a.N);
+  if (a.part) a.part += (size_t)pl.head * a.N;
+  return esm::launch_q8_linear(a, st);
 }
 
 #ifndef ESM_SOURCE_HASH
@@ -610,7 +643,7 @@ int q8_linear_ws(const esm_half* x, const uint8_t* q, const esm_half* s, const e
   if (sb && !aligned16(sb)) return fail(ESM_ERR_ALIGN, "q8_linear: packed scales must be 16-byte aligned");
   esm::Q8Args a{H(x), q, H(s), H(b), H(y), M, K, N, pl.mtiles, pl.ntiles, pl.splits,
                 pl.splits > 1 ? static_cast<float*>(workspace) : nullptr, sb, nullptr, 0, pl.nb, pl.big};
-  return hip_status(esm::launch_q8_linear(a, (hipStream_t)stream), "q8_linear launch");
+  return hip_status(q8_launch(a, pl, (hipStream_t)stream), "q8_linear launch");
 }
 
 int q8_linear_noalloc(const esm_half* x, const uint8_t* q, const esm_half* s, const esm_half* b, const uint32_t* sb,
@@ -633,7 +666,7 @@ int q8_linear_noalloc(const esm_half* x, const uint8_t* q, const esm_half* s, co
   }
   esm::Q8Args a{H(x), q, H(s), H(b), H(y), M, K, N, pl.mtiles, pl.ntiles, pl.splits, part,
                 sb, nullptr, 0, pl.nb, pl.big};
-  return hip_status(esm::launch_q8_linear(a, (hipStream_t)stream), "q8_linear_noalloc launch");
+  return hip_status(q8_launch(a, pl, (hipStream_t)stream), "q8_linear_noalloc launch");
 }
 
 size_t q8_linear_partials_bytes(int M, int K, int N) {
@@ -657,7 +690,7 @@ int q8_linear_partials(const esm_half* x, const uint8_t* q, const esm_half* s, c
   *splits = pl.splits;
   esm::Q8Args a{H(x), q, H(s), H(b), nullptr, M, K, N, pl.mtiles, pl.ntiles, pl.splits, parts,
                 sb, nullptr, 0, pl.nb, pl.big};
-  return hip_status(esm::launch_q8_linear(a, (hipStream_t)stream), "q8_linear_partials launch");
+  return hip_status(q8_launch(a, pl, (hipStream_t)stream), "q8_linear_partials launch");
 }
 
 int q8_linear_packed_ws(const esm_half* x, const uint8_t* qp, const uint32_t* sb, esm_half* y, int M, int K, int N,
@@ -681,7 +714,7 @@ int q8_linear_packed_ws(const esm_half* x, const uint8_t* qp, const uint32_t* sb
   }
   esm::Q8Args a{H(x), nullptr, nullptr, nullptr, H(y), M, K, N, pl.mtiles, pl.ntiles, pl.splits,
                 pl.splits > 1 ? static_cast<float*>(workspace) : nullptr, sb, qp, 0, pl.nb, pl.big};
-  return hip_status(esm::launch_q8_linear(a, (hipStream_t)stream), "q8_linear_packed_ws launch");
+  return hip_status(q8_launch(a, pl, (hipStream_t)stream), "q8_linear_packed_ws launch");
 }
 
 int q8_linear_swiglu_packed_ws(const esm_half* x, const uint8_t* qp, const uint32_t* sb, esm_half* y, int M, int K,
@@ -709,7 +742,7 @@ int q8_linear_swiglu_packed_ws(const esm_half* x, const uint8_t* qp, const uint3
   }
   esm::Q8Args a{H(x), nullptr, nullptr, nullptr, H(y), M, K, N, pl.mtiles, pl.ntiles, pl.splits,
                 pl.splits > 1 ? static_cast<float*>(workspace) : nullptr, sb, qp, 1, pl.nb, pl.big};
-  return hip_status(esm::launch_q8_linear(a, (hipStream_t)stream), "q8_linear_swiglu_packed_ws launch");
+  return hip_status(q8_launch(a, pl, (hipStream_t)stream), "q8_linear_swiglu_packed_ws launch");
 }
 
 int q8_linear_packed_partials(const esm_half* x, const uint8_t* qp, const uint32_t* sb, float* parts,
@@ -731,7 +764,7 @@ int q8_linear_packed_partials(const esm_half* x, const uint8_t* qp, const uint32
   *splits = pl.splits;
   esm::Q8Args a{H(x), nullptr, nullptr, nullptr, nullptr, M, K, N, pl.mtiles, pl.ntiles, pl.splits, parts,
                 sb, qp, 0, pl.nb, pl.big};
-  return hip_status(esm::launch_q8_linear(a, (hipStream_t)stream), "q8_linear_packed_partials launch");
+  return hip_status(q8_launch(a, pl, (hipStream_t)stream), "q8_linear_packed_partials launch");
 }
 
 int q8_linear(const esm_half* x, const uint8_t* q, const esm_half* s, const esm_half* b, esm_half* y, int M, int K,

@@ -284,7 +284,9 @@ def test_q8_swiglu_fused_same_bits(gpu_lib, pkg, M, K, N):
     (769, 2560, 2560 * 4),    # a last row tile of one row, SwiGLU pairs in the epilogue
     (1100, 5120, 2560),       # K split, 33 MB of partials
     (1024, 4160, 2624),       # an odd number of K groups, a last weight tile of 64 rows, split
-    (2049, 448, 10240),       # 7 groups: fewer steps than the pipeline is deep, unsplit
+    (2049, 448, 10240),       # 7 groups: fewer steps than the pipeline is deep; the last row on 64-row tiles
+    (1300, 320, 7744),        # 20 rows beyond a whole round on 64-row tiles, a last weight tile of 64 rows
+    (1100, 2560, 2560 * 4),   # 76 of them, SwiGLU pairs in both
 ])
 def test_q8_many_rows(gpu_lib, pkg, M, K, N):
     # 256-row tiles (the plan's choice here) against the fp64 product of the same fp16 weights; packed or not and
