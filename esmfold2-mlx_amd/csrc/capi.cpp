@@ -135,8 +135,8 @@ Q8Plan q8_plan_big(int M, int K, int N, double* cost) {
     }
   }
   // Where the tiles leave a last round mostly empty: whole rounds of them, then the remaining rows on 64-row
-  // tiles in a launch of their own, if the estimate is lower (2560 -> 10240 at M = 1100 107 -> 78 us, at 2200 154 -> 135;
-  // 2560 -> 7680 at M = 1300 91 -> 76, at 1500 110 -> 78).
+  // tiles in a launch of their own, if the estimate is lower (2560 -> 10240 at M = 1100 107 -> 78 us, at
+  // 2200 154 -> 135; 2560 -> 7680 at M = 1300 91 -> 76, at 1500 110 -> 78).
   const long long rows = tiles / cus * cus / p.ntiles * esm::kQ8BigM;
   if (rows > 0 && rows < M) {
     Q8Plan rest = q8_plan_nb(M - (int)rows, K, N, p.nb);

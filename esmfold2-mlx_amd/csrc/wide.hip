@@ -1,6 +1,7 @@
 // Wide path: the triangle update and the pair transition at pair widths other than the
 // 128 channels the per-cell kernels (a), (c) and (e) are specialised for (ESMFold2's real
-// trunk is 256 wide, mlx_trunk.py:3-5). The same arithmetic, split into generic pieces:
+// trunk is 256 wide, mlx_trunk.py:3-5). The same arithmetic, split into generic pieces (at 256 channels the
+// kernels of stream.hip run instead on grids large enough for them):
 //
 //   ln_rows        out[row] = fp16(LN(in[row]))  over C = 128 NCH channels (fp32 statistics)
 //   ln_cf_to_cl    y[cell][ch] = fp16(LN over ch of x[ch][cell]): the contraction's
