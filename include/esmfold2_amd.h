@@ -169,7 +169,9 @@ int tmu_epilogue(const esm_half* x, int ldx, const esm_half* z, const esm_half* 
  * Supported: C = c = 128 (kernels (a), (b), (c)), or C = c a multiple of 128 up to 512
  * (ESMFold2's trunk is 256 wide, mlx_trunk.py:3-5): the wide path, five launches with
  * the same arithmetic (LN_in(z) -> gated projection stored channel-major -> kernel (b)
- * -> LN_mix over channels turned cell-major -> emit and gate GEMMs with the residual).
+ * -> LN_mix over channels turned cell-major -> emit and gate GEMMs with the residual); at
+ * C = 256 on grids that fill the chip three, the LayerNorms inside the projection and the
+ * emit / gate step.
  * L <= 4096 and B * c <= 65535; B * L * L * C is bounded only by memory (each kernel
  * addresses its tile or channel plane from a 64-bit base).
  */
