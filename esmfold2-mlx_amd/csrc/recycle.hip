@@ -113,7 +113,11 @@ __global__ __launch_bounds__(256, 1) void parcae_step_kernel(ParcaeArgs p) {
       for (int t = 0; t < NCH; t++) {
         half8 o;
 #pragma unroll
-        for (int e = 0; e < 8; e++) o[e] = (half_t)(v[t][e] * rstd * g[t][e] + bb[t][e]);
+        for (int e = 0; e < 8; e++) {
+          float y = v[t][e] * rstd * g[t][e] + bb[t][e];
+          __asm__ volatile("" : "+v"(y));  // fp32 then fp16 in every copy of this code: a cell's bits do not depend on its place
+          o[e] = (half_t)y;
+        }
         st16(&n_s[cl * NSTR + 8 * (l16 + 16 * t)], o);
       }
     }

@@ -34,6 +34,27 @@ def test_parcae_step(gpu_lib, pkg, L, inplace):
     assert float((out.double().cpu() - ref).abs().max()) <= 1e-2 * float(inj.pow(2).mean().sqrt())
 
 
+@pytest.mark.parametrize("C", [128, 256])
+@pytest.mark.parametrize("B,L", [(1, 40), (1, 90), (1, 91), (1, 130), (2, 119), (1, 239)])
+def test_parcae_step_does_not_depend_on_the_cell(gpu_lib, pkg, B, L, C):
+    # 16 different cells, over and over: their results are the same bits wherever a cell's tile of 32 stands and in
+    # either half of it (one tile per workgroup up to L = 90 on 256 CUs, two, four and seven rounds, a cut last
+    # tile), and they are the oracle's. 4 sets of them, so that a rounding that differs somewhere shows
+    g = torch.Generator().manual_seed(C + L)
+    w, b = 1 + 0.1 * torch.randn(C, generator=g), 0.1 * torch.randn(C, generator=g)
+    a, bm = torch.rand(C, generator=g), (torch.randn(C, C, generator=g) * C ** -0.5).half()
+    n = B * L * L
+    over = lambda t: t.repeat((n + 15) // 16, 1)[:n].contiguous()  # noqa: E731
+    for _ in range(4):
+        z, zi, rf = (torch.randn(16, C, generator=g) for _ in range(3))
+        zd, zid, rfd = (over(t.to(DEV)).view(B, L, L, C) for t in (z, zi, rf))
+        out = pkg.kernels.parcae_step(zd, zid, rfd, w.to(DEV), b.to(DEV), 1e-5, a.to(DEV), bm.to(DEV)).view(n, C)
+        assert torch.equal(out, over(out[:16]))
+        ref = orc.parcae_step(z.double(), zi.double(), rf.double(), w.double(), b.double(), a.double(), bm.double())
+        inj = ref - a.double() * z.double()
+        assert float((out[:16].double().cpu() - ref).abs().max()) <= 1e-2 * float(inj.pow(2).mean().sqrt())
+
+
 @pytest.mark.parametrize("L,nbins", [(1, 64), (5, 64), (130, 64), (37, 128)])
 def test_expected_distance(gpu_lib, pkg, L, nbins):
     g = torch.Generator().manual_seed(L + nbins)
