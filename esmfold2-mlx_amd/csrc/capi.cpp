@@ -1041,11 +1041,15 @@ int parcae_step(const float* z, const float* z_init, const float* refined, const
     return fail(ESM_ERR_ALIGN, "parcae_step: z, z_init, refined, z_out, b_mat must be 16-byte aligned");
   const size_t ntiles = (ncells + 31) / 32;
   esm::ParcaeArgs args{z, z_init, refined, ln_w, ln_b, eps, a, H(b_mat), z_out, ncells, (int)ntiles, C};
-  // one workgroup per CU, its next tile's loads in flight (two: C = 256 59 against 52 us at L = 238, C = 128 27
-  // against 25)
-  const size_t cap = (size_t)cu_count();
+  // At C = 128, from two tiles per CU on, two workgroups per CU run their phases against each other; below that
+  // (and at C = 256, whose registers fill a SIMD: two 59 us, one 52 at L = 238) one per CU has its next tile's
+  // loads in flight. us, one / two, inputs in cache: L = 238 20.4 / 20.3, L = 280 27.4 / 26.0, L = 340 38.9 / 36.7;
+  // not in cache: L = 100 (313 tiles on 256 CUs) 9.1 / 9.7, L = 120 (450) 9.7 / 9.7, L = 128 (512) 9.9 / 9.9,
+  // L = 200 20.1 / 19.9, L = 238 25.5 / 25.5, L = 512 98.2 / 99.0.
+  const bool ahead = C == 256 || ntiles < 2 * (size_t)cu_count();
+  const size_t cap = (size_t)cu_count() * (ahead ? 1 : 2);
   const int grid = (int)(ntiles < cap ? ntiles : cap);
-  return hip_status(esm::launch_parcae_step(args, grid, (hipStream_t)stream), "parcae_step launch");
+  return hip_status(esm::launch_parcae_step(args, grid, ahead, (hipStream_t)stream), "parcae_step launch");
 }
 
 int distogram_expected_distance(const float* r, const esm_half* w, const float* bias, const float* centers, float* ed,

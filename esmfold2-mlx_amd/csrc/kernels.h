@@ -218,7 +218,8 @@ hipError_t launch_emit_stream(const EpilogueArgs& a, hipStream_t s);
 // The whole transition at C = 256, H a multiple of 32 (a.ntiles is set by the launcher).
 hipError_t launch_transition_stream(const TransitionArgs& a, int C, int cus, hipStream_t s);
 hipError_t launch_esmc_ln(const EsmcLnArgs& a, hipStream_t s);
-hipError_t launch_parcae_step(const ParcaeArgs& a, int grid, hipStream_t s);
+// ahead: one workgroup per CU with the next tile's loads in flight (the only form at C = 256).
+hipError_t launch_parcae_step(const ParcaeArgs& a, int grid, bool ahead, hipStream_t s);
 hipError_t launch_expected_distance(const DistoArgs& a, int grid, hipStream_t s);
 // ws: abs_diff_quantile_ws_size(n) bytes (0: none needed), or nullptr (one workgroup whatever n).
 size_t abs_diff_quantile_ws_size(size_t n);

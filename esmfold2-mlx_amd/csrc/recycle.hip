@@ -16,12 +16,13 @@ namespace esm {
 // holding the 8-channel chunks l + 16 t, fp32 statistics) into LDS as fp16, one barrier,
 // D[co][cell] = B[co][:] . LN(u)[cell][:] (fp32 accumulation), then a[co] * z + D in fp32,
 // 16-byte stores (4 consecutive channels per lane and quad).
-// Bound by its four fp32 streams (232 MB at L=238, C=256). All loads of the next tile, z's too, are in flight
-// while a tile computes (96 registers per set at C = 256); with z loaded behind the products and u at the top
-// of its own tile, on inputs the cache does not hold: 58 -> 52 us at L=238 (4.5 TB/s), 224 -> 196 us at L=512;
-// C=128 25.8 -> 26.2 and 104 -> 98 us.
-template <int CC>
-__global__ __launch_bounds__(256, 1) void parcae_step_kernel(ParcaeArgs p) {
+// Bound by its four fp32 streams (232 MB at L=238, C=256). AHEAD: all loads of the next tile, z's too, are in
+// flight while a tile computes (96 registers per set at C = 256); with z loaded behind the products and u at the
+// top of its own tile, on inputs the cache does not hold: 57 -> 52 us at L=238 (4.5 TB/s), 224 -> 196 us at
+// L=512. Otherwise (C = 128) two workgroups per CU, each with all of a tile's loads at its top: against z
+// loaded behind the products 34.9 -> 33.8 us at L=280, 104.6 -> 99.0 at L=512.
+template <int CC, bool AHEAD>
+__global__ __launch_bounds__(256, AHEAD ? 1 : 2) void parcae_step_kernel(ParcaeArgs p) {
   constexpr int OB = CC / 128;       // 32-channel output blocks per wave
   constexpr int NCH = CC / 128;      // 8-channel chunks per lane in the LayerNorm
   constexpr int NSTR = CC + 8;       // LDS row stride (halfs) of the LayerNormed tile
@@ -146,10 +147,17 @@ __global__ __launch_bounds__(256, 1) void parcae_step_kernel(ParcaeArgs p) {
       }
     __syncthreads();  // n_s is rewritten by the next tile
   };
-  // The next tile's loads are in flight while this one computes, in two register sets (no copy waits on a load).
   const int G = gridDim.x;
   Loads l0, l1;
   int tile = blockIdx.x;
+  if constexpr (!AHEAD) {
+    for (; tile < p.ntiles; tile += G) {
+      load(l0, tile);
+      process(l0, tile);
+    }
+    return;
+  }
+  // The next tile's loads are in flight while this one computes, in two register sets (no copy waits on a load).
   load(l0, tile);
   if (p.ntiles <= G) {  // one tile each: nothing to keep in flight
     process(l0, tile);
@@ -781,11 +789,13 @@ __global__ __launch_bounds__(SQT) void quantile_final_kernel(const SpreadWs* ws,
   }
 }
 
-hipError_t launch_parcae_step(const ParcaeArgs& a, int grid, hipStream_t s) {
-  if (a.C == 128)
-    ESM_LAUNCH(parcae_step_kernel<128>, dim3(grid), dim3(256), 0, s, a);
+hipError_t launch_parcae_step(const ParcaeArgs& a, int grid, bool ahead, hipStream_t s) {
+  if (a.C == 128 && ahead)
+    ESM_LAUNCH((parcae_step_kernel<128, true>), dim3(grid), dim3(256), 0, s, a);
+  else if (a.C == 128)
+    ESM_LAUNCH((parcae_step_kernel<128, false>), dim3(grid), dim3(256), 0, s, a);
   else if (a.C == 256)
-    ESM_LAUNCH(parcae_step_kernel<256>, dim3(grid), dim3(256), 0, s, a);
+    ESM_LAUNCH((parcae_step_kernel<256, true>), dim3(grid), dim3(256), 0, s, a);
   else
     return hipErrorInvalidValue;
   return hipGetLastError();

@@ -35,11 +35,12 @@ def test_parcae_step(gpu_lib, pkg, L, inplace):
 
 
 @pytest.mark.parametrize("C", [128, 256])
-@pytest.mark.parametrize("B,L", [(1, 40), (1, 90), (1, 91), (1, 130), (2, 119), (1, 239)])
+@pytest.mark.parametrize("B,L", [(1, 40), (1, 90), (1, 91), (1, 127), (1, 128), (1, 130), (2, 119), (1, 239)])
 def test_parcae_step_does_not_depend_on_the_cell(gpu_lib, pkg, B, L, C):
     # 16 different cells, over and over: their results are the same bits wherever a cell's tile of 32 stands and in
     # either half of it (one tile per workgroup up to L = 90 on 256 CUs, two, four and seven rounds, a cut last
-    # tile), and they are the oracle's. 4 sets of them, so that a rounding that differs somewhere shows
+    # tile; at C = 128 two workgroups per CU from L = 128 on), and they are the oracle's. 4 sets of them, so that
+    # a rounding that differs somewhere shows
     g = torch.Generator().manual_seed(C + L)
     w, b = 1 + 0.1 * torch.randn(C, generator=g), 0.1 * torch.randn(C, generator=g)
     a, bm = torch.rand(C, generator=g), (torch.randn(C, C, generator=g) * C ** -0.5).half()
