@@ -7,6 +7,7 @@ torch, passes raw pointers plus the current HIP stream, and raises
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 
 import torch
@@ -14,6 +15,7 @@ import torch
 from . import capi, scratch
 
 F16 = torch.float16
+_UNGUARDED = contextlib.nullcontext()  # for a call that does not touch the shared scratch
 
 
 def _dev(t: torch.Tensor, name: str, dtype=None) -> torch.Tensor:
@@ -118,10 +120,11 @@ def transition(z, ln_w, ln_b, eps, w1, w3, w2=None, out=None):
         raise capi.EsmError(-2, f"transition: w1 {tuple(w1.shape)}, w3 {tuple(w3.shape)} for C={C}")
     out = torch.empty_like(z) if out is None else _out(out, "out", F16, z.numel())
     need = int(lib.pair_transition_workspace_bytes(B, L, C, H, int(w2 is not None)))
-    ws = scratch.get(need, z.device) if need else None  # the wide path's LN(z) and hidden planes
-    capi.check(lib.pair_transition_ws(z.data_ptr(), out.data_ptr(), _dev(ln_w, "ln_w", torch.float32).data_ptr(),
-                                      _dev(ln_b, "ln_b", torch.float32).data_ptr(), float(eps), w1.data_ptr(),
-                                      _ptr(w2), w3.data_ptr(), B, L, C, H, _ptr(ws), need, capi.stream_ptr()))
+    with scratch.guard(z.device) if need else _UNGUARDED:
+        ws = scratch.get(need, z.device) if need else None  # the wide path's LN(z) and hidden planes
+        capi.check(lib.pair_transition_ws(z.data_ptr(), out.data_ptr(), _dev(ln_w, "ln_w", torch.float32).data_ptr(),
+                                          _dev(ln_b, "ln_b", torch.float32).data_ptr(), float(eps), w1.data_ptr(),
+                                          _ptr(w2), w3.data_ptr(), B, L, C, H, _ptr(ws), need, capi.stream_ptr()))
     return out
 
 
@@ -139,9 +142,6 @@ def esmc_layer_norm(x, w, b, eps, y=None, alpha: float = 1.0, x_out=None, out=No
         _out(y, "y", F16, M * D)
     if y_parts is not None:
         _dev(y_parts[0], "y_parts", torch.float32)
-        gen = getattr(y_parts, "generation", None)
-        if gen is not None:  # partials living in the shared scratch: not overwritten since
-            scratch.check_generation(gen, y_parts[0].device, "esmc_layer_norm: y_parts")
         if y_parts[0].numel() < int(y_parts[1]) * M * D:
             raise capi.EsmError(-2, "esmc_layer_norm: y_parts smaller than splits x M x D")
     if y is not None or y_parts is not None:
@@ -151,8 +151,12 @@ def esmc_layer_norm(x, w, b, eps, y=None, alpha: float = 1.0, x_out=None, out=No
     wp, bp = _dev(w, "w", torch.float32).data_ptr(), None if b is None else _dev(b, "b", torch.float32).data_ptr()
     hp, h32 = (None, out.data_ptr()) if fp32_out else (out.data_ptr(), None)
     if y_parts is not None:
-        capi.check(lib.esmc_layer_norm_parts(x.data_ptr(), y_parts[0].data_ptr(), int(y_parts[1]), float(alpha),
-                                             _ptr(x_out), wp, bp, float(eps), hp, h32, M, D, capi.stream_ptr()))
+        gen = getattr(y_parts, "generation", None)  # partials living in the shared scratch: not overwritten since
+        with _UNGUARDED if gen is None else scratch.guard(y_parts[0].device):
+            if gen is not None:
+                scratch.check_generation(gen, y_parts[0].device, "esmc_layer_norm: y_parts")
+            capi.check(lib.esmc_layer_norm_parts(x.data_ptr(), y_parts[0].data_ptr(), int(y_parts[1]), float(alpha),
+                                                 _ptr(x_out), wp, bp, float(eps), hp, h32, M, D, capi.stream_ptr()))
     else:
         capi.check(lib.esmc_layer_norm(x.data_ptr(), _ptr(y), float(alpha), _ptr(x_out), wp, bp, float(eps), hp, h32,
                                        M, D, capi.stream_ptr()))
@@ -234,10 +238,11 @@ def esmc_block(x, h, norms, linears, next_w, next_b, eps, alpha: float, B: int, 
         lin.append(_weight(codes, n + " codes", torch.uint8, N * K))
         lin.append(_weight(packed, n + " packed", torch.int32, N * K // 16))
     need = int(lib.esmc_block_workspace_bytes(M, n_heads, F))
-    ws, wp, stream = scratch.take(need, x.device)
-    capi.check(lib.esmc_block(x.data_ptr(), h.data_ptr(), sid, *ln, *lin, float(eps), float(alpha), float(base),
-                              x_out.data_ptr(), None if fp32 else out.data_ptr(), out.data_ptr() if fp32 else None, B,
-                              L, n_heads, F, wp, need, stream))
+    with scratch.guard(x.device):
+        ws, wp, stream = scratch.take(need, x.device)
+        capi.check(lib.esmc_block(x.data_ptr(), h.data_ptr(), sid, *ln, *lin, float(eps), float(alpha), float(base),
+                                  x_out.data_ptr(), None if fp32 else out.data_ptr(),
+                                  out.data_ptr() if fp32 else None, B, L, n_heads, F, wp, need, stream))
 
 
 def parcae_step(z, z_init, refined, ln_w, ln_b, eps, a, b_mat, out=None):
@@ -469,11 +474,9 @@ def q8_linear_packed(x, codes, packed, N: int, group: int = 64):
     sb = _weight(packed, "packed", torch.int32, int(lib.q8_packed_scales_bytes(N, K)))
     y = torch.empty(M, N, dtype=F16, device=x.device)
     need = int(lib.q8_linear_workspace_bytes(M, K, N))
-    if need:
-        ws, wp, stream = scratch.take(need, x.device)
-    else:
-        ws, wp, stream = None, None, capi.stream_ptr()
-    capi.check(lib.q8_linear_packed_ws(x.data_ptr(), qp, sb, y.data_ptr(), M, K, N, group, wp, need, stream))
+    with scratch.guard(x.device) if need else _UNGUARDED:
+        ws, wp, stream = scratch.take(need, x.device) if need else (None, None, capi.stream_ptr())
+        capi.check(lib.q8_linear_packed_ws(x.data_ptr(), qp, sb, y.data_ptr(), M, K, N, group, wp, need, stream))
     return y
 
 

@@ -61,8 +61,9 @@ class Q8Linear(nn.Module):
         x2 = x.reshape(-1, self.in_features).to(torch.float16).contiguous()
         M = x2.shape[0]
         n = kernels.q8_workspace_bytes(M, self.in_features, self.out_features)
-        ws = scratch.get(n, x2.device) if n else None
-        y = kernels.q8_linear_swiglu(x2, self.codes_packed, self.packed, self.out_features, GROUP, workspace=ws)
+        with scratch.guard(x2.device):
+            ws = scratch.get(n, x2.device) if n else None
+            y = kernels.q8_linear_swiglu(x2, self.codes_packed, self.packed, self.out_features, GROUP, workspace=ws)
         return y.reshape(*lead, self.out_features // 2)
 
     def _layouts(self):
@@ -98,8 +99,9 @@ class Q8Linear(nn.Module):
         x2 = x.reshape(-1, self.in_features).to(torch.float16).contiguous()
         M = x2.shape[0]
         n = kernels.q8_workspace_bytes(M, self.in_features, self.out_features)
-        ws = scratch.get(n, x2.device) if n else None  # split-K partials, only while this call runs
-        y = kernels.q8_linear(x2, self.q, self.scales, self.biases, GROUP, workspace=ws, packed=sb, codes=qp)
+        with scratch.guard(x2.device):
+            ws = scratch.get(n, x2.device) if n else None  # split-K partials, only while this call runs
+            y = kernels.q8_linear(x2, self.q, self.scales, self.biases, GROUP, workspace=ws, packed=sb, codes=qp)
         y = y.reshape(*lead, self.out_features)
         return y if x.dtype == torch.float16 else y.to(x.dtype)
 
@@ -112,11 +114,12 @@ class Q8Linear(nn.Module):
         once the scratch has been handed out again."""
         x2 = x.reshape(-1, self.in_features).to(torch.float16).contiguous()
         M = x2.shape[0]
-        buf = scratch.get(kernels.q8_partials_bytes(M, self.in_features, self.out_features), x2.device)
-        gen = scratch.generation(x2.device)
         sb, qp = self._layouts()
-        parts, splits = kernels.q8_linear_partials(x2, self.q, self.scales, self.biases, buf, GROUP, packed=sb,
-                                                   codes=qp)
+        with scratch.guard(x2.device):
+            buf = scratch.get(kernels.q8_partials_bytes(M, self.in_features, self.out_features), x2.device)
+            gen = scratch.generation(x2.device)
+            parts, splits = kernels.q8_linear_partials(x2, self.q, self.scales, self.biases, buf, GROUP, packed=sb,
+                                                       codes=qp)
         return ScratchParts(parts, splits, gen)
 
 

@@ -11,12 +11,15 @@ Rules:
     the buffer is recorded on it (``Tensor.record_stream``), so when a grown buffer replaces
     it the caching allocator keeps the old memory until the work queued on each of those
     streams is done.
-  * Calls on one device are ordered through the buffer: when ``get`` is called on a stream
+  * Calls on one device are ordered through the buffer: a user holds ``guard(device)`` from its
+    ``get`` until the launches that touch the bytes are queued, so two threads never interleave
+    theirs (a native call runs without the interpreter lock). When ``get`` is called on a stream
     other than the buffer's last user, that stream first waits for the work already queued on
     the last user (``wait_stream``), so two streams never run their scratch users at once.
     Under HIP-graph capture no wait is recorded (the caller orders the capture).
   * Each ``get`` starts a new generation: a view handed out earlier (``Q8Linear.partials``)
-    is valid only until the next ``get`` on that device, which ``check_generation`` tells.
+    is valid only until the next ``get`` on that device, which ``check_generation`` tells (the
+    consumer holds the guard from that check until it is queued).
   * A HIP graph that captured calls keeps the buffers they used alive: ``current`` gives
     the buffer to hold next to the graph.
 """
@@ -40,6 +43,7 @@ class _Slot:
 
 
 _slots: dict[int, _Slot] = {}
+_guards: dict[int, threading.RLock] = {}
 
 
 def _index(device) -> int:
@@ -47,6 +51,13 @@ def _index(device) -> int:
     if d.type != "cuda":
         raise ValueError(f"scratch lives in device memory, got {d}")
     return torch.cuda.current_device() if d.index is None else d.index
+
+
+def guard(device=None) -> threading.RLock:
+    """The lock that a user of the device's scratch holds from its ``get`` until its launches are queued."""
+    idx = _index(device)
+    g = _guards.get(idx)
+    return _guards.setdefault(idx, threading.RLock()) if g is None else g
 
 
 def _claim(nbytes: int, device):
@@ -74,7 +85,8 @@ def _claim(nbytes: int, device):
 
 
 def get(nbytes: int, device=None) -> torch.Tensor:
-    """A uint8 view of ``nbytes`` (>= 1) at a 256-byte aligned address of the device's scratch."""
+    """A uint8 view of ``nbytes`` (>= 1) at a 256-byte aligned address of the device's scratch, for a caller
+    that holds ``guard(device)`` until the launches that use it are queued."""
     buf, _ = _claim(nbytes, device)
     off = (-buf.data_ptr()) % ALIGN
     return buf[off:off + max(int(nbytes), 1)]
@@ -82,7 +94,7 @@ def get(nbytes: int, device=None) -> torch.Tensor:
 
 def take(nbytes: int, device=None):
     """``get`` for one launch: (buffer, 256-byte aligned address in it, raw stream). The caller holds the
-    buffer until its launches are queued."""
+    buffer and ``guard(device)`` until its launches are queued."""
     buf, stream = _claim(nbytes, device)
     return buf, (buf.data_ptr() + ALIGN - 1) // ALIGN * ALIGN, stream.cuda_stream
 

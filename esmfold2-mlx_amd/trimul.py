@@ -83,7 +83,8 @@ class TriMul(nn.Module):
     # --- forward -----------------------------------------------------------------------------
     def workspace(self, B: int, L: int, device) -> torch.Tensor:
         """The a, b, x planes of one call: a 256-byte aligned view of the device's shared scratch
-        (every update of a trunk runs in the same bytes, one after another)."""
+        (every update of a trunk runs in the same bytes, one after another). Taken and used under
+        ``scratch.guard(device)``."""
         return scratch.get(capi.lib().tmu_workspace_bytes(B, L, self.c), device)
 
     def run(self, z16: torch.Tensor, mask16: torch.Tensor | None, out: torch.Tensor, residual: bool) -> torch.Tensor:
@@ -92,13 +93,15 @@ class TriMul(nn.Module):
         B, L, _, C = z16.shape
         if tuple(out.shape) != tuple(z16.shape) or out.dtype != F16 or not out.is_contiguous():
             raise capi.EsmError(-2, f"out must be a contiguous fp16 {tuple(z16.shape)} tensor")
-        ws = self.workspace(B, L, z16.device)
-        capi.check(lib.tmu_forward_ws(z16.data_ptr(), None if mask16 is None else mask16.data_ptr(),
-                                      self.ln_in_w.data_ptr(), self.ln_in_b.data_ptr(), self.ln_in_eps,
-                                      self.w_bundle.data_ptr(), self.ln_mix_w.data_ptr(), self.ln_mix_b.data_ptr(),
-                                      self.ln_mix_eps, self.w_emit.data_ptr(), self.w_gate.data_ptr(),
-                                      out.data_ptr(), ws.data_ptr(), ws.numel(), B, L, C, self.c,
-                                      int(self.outgoing), int(residual), int(self.out_mask), capi.stream_ptr()))
+        with scratch.guard(z16.device):
+            ws = self.workspace(B, L, z16.device)
+            capi.check(lib.tmu_forward_ws(z16.data_ptr(), None if mask16 is None else mask16.data_ptr(),
+                                          self.ln_in_w.data_ptr(), self.ln_in_b.data_ptr(), self.ln_in_eps,
+                                          self.w_bundle.data_ptr(), self.ln_mix_w.data_ptr(),
+                                          self.ln_mix_b.data_ptr(), self.ln_mix_eps, self.w_emit.data_ptr(),
+                                          self.w_gate.data_ptr(), out.data_ptr(), ws.data_ptr(), ws.numel(), B, L, C,
+                                          self.c, int(self.outgoing), int(residual), int(self.out_mask),
+                                          capi.stream_ptr()))
         return out
 
     def forward(self, pair_grid: torch.Tensor, visibility: torch.Tensor | None = None,
@@ -148,12 +151,13 @@ class TriMulPair(nn.Module):
 def run_pair(o: TriMul, i: TriMul, z16: torch.Tensor, mask16: torch.Tensor | None, out: torch.Tensor) -> torch.Tensor:
     """out = z1 + i(z1), z1 = z16 + o(z16) on the current stream (fp16; ``out`` may be ``z16``)."""
     B, L = z16.shape[0], z16.shape[1]
-    ws = o.workspace(B, L, z16.device)
-    capi.check(capi.lib().tmu_pair_forward_ws(
-        z16.data_ptr(), None if mask16 is None else mask16.data_ptr(),
-        o.ln_in_w.data_ptr(), o.ln_in_b.data_ptr(), o.ln_in_eps, o.w_bundle.data_ptr(), o.ln_mix_w.data_ptr(),
-        o.ln_mix_b.data_ptr(), o.ln_mix_eps, o.w_emit.data_ptr(), o.w_gate.data_ptr(), int(o.out_mask),
-        i.ln_in_w.data_ptr(), i.ln_in_b.data_ptr(), i.ln_in_eps, i.w_bundle.data_ptr(), i.ln_mix_w.data_ptr(),
-        i.ln_mix_b.data_ptr(), i.ln_mix_eps, i.w_emit.data_ptr(), i.w_gate.data_ptr(), int(i.out_mask),
-        out.data_ptr(), ws.data_ptr(), ws.numel(), B, L, o.C, o.c, capi.stream_ptr()))
+    with scratch.guard(z16.device):
+        ws = o.workspace(B, L, z16.device)
+        capi.check(capi.lib().tmu_pair_forward_ws(
+            z16.data_ptr(), None if mask16 is None else mask16.data_ptr(),
+            o.ln_in_w.data_ptr(), o.ln_in_b.data_ptr(), o.ln_in_eps, o.w_bundle.data_ptr(), o.ln_mix_w.data_ptr(),
+            o.ln_mix_b.data_ptr(), o.ln_mix_eps, o.w_emit.data_ptr(), o.w_gate.data_ptr(), int(o.out_mask),
+            i.ln_in_w.data_ptr(), i.ln_in_b.data_ptr(), i.ln_in_eps, i.w_bundle.data_ptr(), i.ln_mix_w.data_ptr(),
+            i.ln_mix_b.data_ptr(), i.ln_mix_eps, i.w_emit.data_ptr(), i.w_gate.data_ptr(), int(i.out_mask),
+            out.data_ptr(), ws.data_ptr(), ws.numel(), B, L, o.C, o.c, capi.stream_ptr()))
     return out
