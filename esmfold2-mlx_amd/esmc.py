@@ -16,10 +16,12 @@ from __future__ import annotations
 import math
 import os
 import re
+from functools import partial
 from types import SimpleNamespace
 
 import torch
 from torch import nn
+from torch.nn.modules.module import _has_any_global_hook
 
 from . import kernels
 from .q8 import Q8Linear
@@ -55,6 +57,18 @@ def hf_layer(tensors, i: int, device=None) -> tuple[dict, dict]:
         w = torch.cat([get(h).detach().float() for h in parts]) if len(parts) > 1 else get(parts[0]).detach().float()
         lin[n] = Q8Linear.from_float(w, device=device)
     return ln, lin
+
+
+_LINEAR_METHODS = (Q8Linear.forward, Q8Linear.partials, Q8Linear.swiglu)
+
+
+def _as_defined(m) -> bool:
+    """Whether a call of this linear runs ``Q8Linear``'s own code and nothing else: no other class, no hook on
+    the module, no method replaced on it."""
+    d = m.__dict__
+    return (type(m) is Q8Linear and "forward" not in d and "partials" not in d and "swiglu" not in d
+            and not (d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"]
+                     or d["_backward_pre_hooks"]))
 
 
 class EsmcBlock(nn.Module):
@@ -120,15 +134,28 @@ class EsmcBlock(nn.Module):
         act = self.w1.swiglu(h2) if self.w1.pair_rows else kernels.esmc_swiglu(self.w1(h2))
         return self.w2.partials(act)
 
+    def _native_linears(self):
+        """The four linears when one native call does what the block's separate calls would do, else None: every
+        linear with its packed layouts and the block's shapes, and nothing put in the place of a part of the block
+        or hooked into it."""
+        lins = (self.wqkv, self.wo, self.w1, self.w2)
+        own = (all(_as_defined(m) for m in lins) and not _has_any_global_hook()
+               and (Q8Linear.forward, Q8Linear.partials, Q8Linear.swiglu) == _LINEAR_METHODS
+               and (getattr(self.attention, "__func__", None), getattr(self.ffn, "__func__", None)) == _BLOCK_METHODS)
+        D, F = self.D, self.F
+        if (own and self.w1.pair_rows and not any(m.pair_rows for m in (self.wqkv, self.wo, self.w2))
+                and F % 320 == 0 and D % 128 == 0 and all(m.codes_packed is not None for m in lins)
+                and [(m.out_features, m.in_features) for m in lins] == [(3 * D, D), (D, D), (2 * F, D), (D, F)]):
+            return lins
+        return None
+
     def run(self, x: torch.Tensor, h: torch.Tensor, sid, res_scale: float, next_w, next_b, x_out: torch.Tensor,
             out: torch.Tensor) -> None:
         """The block on x [B, L, D] fp32 and h = LN1(x): x_out = its output, out = the LayerNorm (next_w, next_b)
-        of that (fp16 or fp32). One native call when every linear has its packed layouts (codes of a width that
-        is a multiple of 128, so that their size says which shape they are), else the separate calls."""
+        of that (fp16 or fp32): one native call or the separate ones (``_native_linears``)."""
         B, L, D = x.shape
-        lins = (self.wqkv, self.wo, self.w1, self.w2)
-        if (self.w1.pair_rows and not any(m.pair_rows for m in (self.wqkv, self.wo, self.w2)) and B and L
-                and self.F % 320 == 0 and D % 128 == 0 and all(m.codes_packed is not None for m in lins)):
+        lins = self._native_linears() if isinstance(self, EsmcBlock) and B and L and D == self.D else None
+        if lins is not None:
             kernels.esmc_block(x, h, (self.q_ln, self.k_ln, self.ln2_w, self.ln2_b),
                                [(m.codes_packed, m.packed) for m in lins], next_w, next_b, EPS, 1.0 / res_scale, B, L,
                                self.n_heads, self.F, x_out, out, sid)
@@ -146,6 +173,9 @@ class EsmcBlock(nn.Module):
         # (the LN output of this call is not needed)
         self.run(x, h, _chain_ids(sequence_id, x.device), res_scale, self.ln1_w, self.ln1_b, out, torch.empty_like(h))
         return out
+
+
+_BLOCK_METHODS = (EsmcBlock.attention, EsmcBlock.ffn)
 
 
 def _chain_ids(sequence_id, device):
@@ -253,11 +283,13 @@ class HipEsmc(nn.Module):
         x_last = torch.empty(B, L, D, dtype=torch.float32, device=dev)
         states = hs.unbind(0)
         for i, blk in enumerate(self.layers):
+            # (another module in a block's place has its attention, ffn and ln1_*, and may have no run)
+            run = blk.run if hasattr(blk, "run") else partial(EsmcBlock.run, blk)
             if i + 1 < n:  # the output into hidden_states[i+1], fused with the next input LN
                 nxt = self.layers[i + 1]
-                blk.run(states[i], h, sid, self.res_scale, nxt.ln1_w, nxt.ln1_b, states[i + 1], h)
+                run(states[i], h, sid, self.res_scale, nxt.ln1_w, nxt.ln1_b, states[i + 1], h)
             else:  # the last block's output is only seen through the final norm (weights only)
-                blk.run(states[i], h, sid, self.res_scale, self.norm_w, None, x_last, states[n])
+                run(states[i], h, sid, self.res_scale, self.norm_w, None, x_last, states[n])
         return hs
 
     def forward(self, input_ids=None, sequence_id=None, output_hidden_states=True, **_):

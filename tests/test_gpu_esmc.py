@@ -230,6 +230,96 @@ def test_native_block_equals_the_separate_calls(gpu_lib, pkg, B, L, D, F_, H, ch
     assert torch.equal(got_x, want_x) and torch.equal(got_h, want_h)
 
 
+def _native_block(pkg, seed=0):
+    """A small block that takes the native call, its input, and its output from there."""
+    D, F_, H, L = 256, 320, 4, 33
+    blk = _module_block(pkg, _weights(D, F_, seed=seed), H)
+    x = (2 * torch.randn(1, L, D, generator=_gen(seed + 1))).to(DEV)
+    before = pkg.scratch.generation(DEV)
+    ref = blk(x)
+    assert pkg.scratch.generation(DEV) == before + 1  # one native call
+    return blk, x, ref
+
+
+def test_block_runs_what_is_hooked_into_its_parts(gpu_lib, pkg):
+    # what a program hooks into a linear of the block, or puts in its place, runs
+    blk, x, ref = _native_block(pkg)
+    calls = []
+    hook = blk.wqkv.register_forward_hook(lambda m, a, y: (calls.append("hook"), y * 0)[1])
+    assert not torch.equal(blk(x), ref) and calls == ["hook"]  # (q, k, v of zeros: another result)
+    hook.remove()
+    hook = blk.wqkv.register_forward_pre_hook(lambda m, a: calls.append("pre"))
+    assert torch.equal(blk(x), ref) and calls == ["hook", "pre"]
+    hook.remove()
+    hook = torch.nn.modules.module.register_module_forward_hook(
+        lambda m, a, y: calls.append("global") if m is blk.wqkv else None)
+    try:
+        assert torch.equal(blk(x), ref) and calls[2:] == ["global"]
+    finally:
+        hook.remove()
+    own = blk.wqkv.forward
+    blk.wqkv.forward = lambda h: (calls.append("forward"), own(h))[1]
+    assert torch.equal(blk(x), ref) and calls[3:] == ["forward"]
+    del blk.wqkv.forward
+
+    class Wrapped(torch.nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner = inner
+
+        def forward(self, h):
+            calls.append("wrapped")
+            return self.inner(h)
+
+    blk.wqkv = Wrapped(blk.wqkv)
+    assert torch.equal(blk(x), ref) and calls[4:] == ["wrapped"]
+    blk.wqkv = blk.wqkv.inner
+    before = pkg.scratch.generation(DEV)
+    assert torch.equal(blk(x), ref) and pkg.scratch.generation(DEV) == before + 1  # as it was
+
+
+def test_block_runs_replaced_methods(gpu_lib, pkg):
+    # an ffn or attention of its own, on the class or on the object; in the whole model too, where a module that is
+    # no EsmcBlock can stand in a block's place
+    blk, x, ref = _native_block(pkg, seed=3)
+    calls, E = [], pkg.esmc.EsmcBlock
+
+    class Own(E):
+        def ffn(self, h2):
+            calls.append("ffn")
+            return super().ffn(h2)
+
+    blk.__class__ = Own
+    assert torch.equal(blk(x), ref) and calls == ["ffn"]
+    blk.__class__ = E
+    attention = blk.attention
+    blk.attention = lambda *a: (calls.append("attention"), attention(*a))[1]
+    assert torch.equal(blk(x), ref) and calls == ["ffn", "attention"]
+    del blk.attention
+
+    class Standing(torch.nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner, self.ln1_w, self.ln1_b = inner, inner.ln1_w, inner.ln1_b
+
+        def attention(self, *a):
+            calls.append("standing")
+            self.inner.attention(*a)
+
+        def ffn(self, h2):
+            return self.inner.ffn(h2)
+
+    g = _gen(8)
+    embed, ids = torch.randn(33, 256, generator=g), torch.randint(0, 33, (1, 20), generator=g).to(DEV)
+    model = pkg.esmc.HipEsmc(embed, [blk, _native_block(pkg, seed=5)[0]], torch.ones(256), n_heads=4)
+    want = model(input_ids=ids).hidden_states
+    for i in range(2):
+        model.layers[i] = Standing(model.layers[i])
+        assert torch.equal(model(input_ids=ids).hidden_states, want) and calls.pop() == "standing"
+        assert calls == ["ffn", "attention"]
+        model.layers[i] = model.layers[i].inner
+
+
 def test_block_graph_replay(gpu_lib, pkg):
     """The block captured as one HIP graph: every replay equals the eager result bit for bit,
     with eager launches of the block between the replays."""
