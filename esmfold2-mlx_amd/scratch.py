@@ -47,7 +47,8 @@ _guards: dict[int, threading.RLock] = {}
 
 
 def _index(device) -> int:
-    d = torch.device(device) if device is not None else torch.device("cuda", torch.cuda.current_device())
+    d = device if type(device) is torch.device else (
+        torch.device(device) if device is not None else torch.device("cuda", torch.cuda.current_device()))
     if d.type != "cuda":
         raise ValueError(f"scratch lives in device memory, got {d}")
     return torch.cuda.current_device() if d.index is None else d.index
@@ -65,10 +66,11 @@ def _claim(nbytes: int, device):
     idx = _index(device)
     need = max(int(nbytes), 1) + ALIGN
     stream = torch.cuda.current_stream(idx)
-    capturing = torch.cuda.is_current_stream_capturing()
     with _lock:
         slot = _slots.get(idx)
-        if slot is not None and slot.stream != stream and not capturing:
+        moved = slot is not None and slot.stream != stream
+        capturing = moved and torch.cuda.is_current_stream_capturing()
+        if moved and not capturing:
             stream.wait_stream(slot.stream)  # the previous user's queued work first
         if slot is None or slot.buf.numel() < need:
             # grow geometrically so a slowly rising size does not reallocate every call; the
@@ -76,7 +78,7 @@ def _claim(nbytes: int, device):
             size = need if slot is None else max(need, slot.buf.numel() + slot.buf.numel() // 4)
             buf = torch.empty(size, dtype=torch.uint8, device=torch.device("cuda", idx))
             slot = _slots[idx] = _Slot(buf, stream, 0 if slot is None else slot.generation)
-        elif slot.stream != stream:
+        elif moved:
             if not capturing:
                 slot.buf.record_stream(stream)
             slot.stream = stream
