@@ -241,6 +241,30 @@ def _native_block(pkg, seed=0):
     return blk, x, ref
 
 
+@pytest.mark.parametrize("F_", [320, 384])
+def test_chain_ids_of_other_shapes(gpu_lib, pkg, F_):
+    # ids whose every row is one chain mean no mask whatever their shape; several chains need [B, L]
+    # (F = 320 is the one-call block, 384 the separate calls)
+    D, H, B, L = 256, 4, 2, 21
+    blk = _module_block(pkg, _weights(D, F_, seed=9), H)
+    embed = torch.randn(33, D, generator=_gen(3))
+    model = pkg.esmc.HipEsmc(embed, [blk], torch.ones(D), n_heads=H)
+    x = (2 * torch.randn(B, L, D, generator=_gen(4))).to(DEV)
+    ids = torch.randint(0, 33, (B, L), generator=_gen(5)).to(DEV)
+    ref, href = blk(x), model(input_ids=ids).hidden_states
+    for sid in (torch.zeros(1, L), torch.tensor([[3], [4]]), torch.arange(B)[:, None].expand(B, L),
+                torch.ones(B, L, 1, dtype=torch.int64), torch.full((1, 1), 7), torch.zeros(B, L + 5, dtype=torch.int32)):
+        assert torch.equal(blk(x, sid), ref), tuple(sid.shape)
+        assert torch.equal(model(input_ids=ids, sequence_id=sid.to(DEV)).hidden_states, href), tuple(sid.shape)
+    two = torch.arange(L).expand(1, L) // 11
+    assert not torch.equal(blk(x, two.expand(B, L)), ref)
+    for sid in (two, torch.zeros(B * L)):  # chains of one row for two, and no rows at all
+        with pytest.raises((pkg.capi.EsmError, IndexError)):
+            blk(x, sid.to(DEV))
+        with pytest.raises((pkg.capi.EsmError, IndexError)):
+            model(input_ids=ids, sequence_id=sid.to(DEV))
+
+
 def test_block_runs_what_is_hooked_into_its_parts(gpu_lib, pkg):
     # what a program hooks into a linear of the block, or puts in its place, runs
     blk, x, ref = _native_block(pkg)
