@@ -109,7 +109,7 @@ double q8_plan_cost(const Q8Plan& p, int M, int K, int N) {
 }
 // The many-rows form: tiles of 256 rows of x by 160 weight rows, its split count the cheapest by the same kind
 // of estimate: a group of 64 k takes ~1.1 us, a workgroup's start and end ~5.5 (the 64-row form's ~6 per round);
-// up to two workgroups per CU where K is split, so that the partials stay under 84 MB on 256 CUs. It is taken
+// up to two workgroups per CU where K is split, so that the partials stay within 80 MiB on 256 CUs. It is taken
 // where its estimate is lower and the scratch at hand holds its partials, and only where those are no fewer bytes
 // than the 64-row form's, so that no call is taken with less scratch than that form needs. Measured at M = 512,
 // 700, 900 and 1100, 64-row form / this, us: 2560 -> 10240 45 / 50, 64 / 51, 87 / 51, 103 / 96 (78 with the row

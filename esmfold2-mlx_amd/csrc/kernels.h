@@ -90,8 +90,9 @@ constexpr int kQ8BigM = 256;  // rows of x per tile of the many-rows form
 constexpr int kQ8TileNbNarrow = 4;
 constexpr int kQ8TileNbWide = 5;
 constexpr int kQ8Waves = 4;
-// Bytes of the device scratch q8_linear_noalloc keeps its split-K partials in.
-constexpr size_t kQ8ScratchBytes = (size_t)16 << 20;
+// Bytes of the device scratch q8_linear_noalloc keeps its split-K partials in: what any plan needs on 256 CUs
+// (two workgroups per CU, each with 256 x 160 fp32 partials).
+constexpr size_t kQ8ScratchBytes = (size_t)80 << 20;
 // The device address of that scratch on the current device (taken once per device).
 hipError_t q8_scratch_address(float** ptr);
 

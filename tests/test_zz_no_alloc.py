@@ -44,6 +44,16 @@ def test_noalloc_matches_workspace_entry_point(gpu_lib, pkg, shapes, packed):
         assert torch.equal(y_na.view(torch.int16), y_ws.view(torch.int16)), f"call {i}: {M}x{K}->{N}"
 
 
+@pytest.mark.parametrize("M,K,N", [(1100, 5120, 2560), (1100, 10240, 2560), (769, 2560, 10240), (1100, 2560, 10240)])
+def test_noalloc_matches_with_many_rows(gpu_lib, pkg, M, K, N):
+    # 256-row tiles: K split with 34 MB of partials, unsplit, and rows divided between two tile forms
+    x, q, s, b = _inputs(pkg, M, K, N, seed=M + K)
+    sb = pkg.kernels.q8_pack_scales(s, b)
+    y_ws = pkg.kernels.q8_linear(x, q, s, b, workspace=pkg.kernels.q8_workspace(M, K, N, device=DEV), packed=sb)
+    y_na = _noalloc(pkg, gpu_lib, x, q, s, b, sb)
+    assert torch.equal(y_na.view(torch.int16), y_ws.view(torch.int16))
+
+
 def test_noalloc_allocates_nothing(gpu_lib, pkg):
     # after a first call (which loads nothing new), further calls leave torch's device memory
     # untouched except for the outputs the caller allocated
