@@ -230,6 +230,78 @@ def test_native_block_equals_the_separate_calls(gpu_lib, pkg, B, L, D, F_, H, ch
     assert torch.equal(got_x, want_x) and torch.equal(got_h, want_h)
 
 
+@pytest.mark.parametrize("L,F_", [(33, 320), (700, 5120), (1100, 5120)])
+def test_native_block_many_rows_and_in_place(gpu_lib, pkg, L, F_):
+    # the LayerNorm behind the block written over its input's, as the model's loop does; at 700 rows some linears
+    # run 256-row tiles, at 1,100 they divide their rows between two forms and w2 splits K over 34 MB of partials
+    H = 40 if F_ == 5120 else 4
+    blk = _module_block(pkg, _weights(64 * H, F_, seed=L), H)
+    x = (2 * torch.randn(1, L, 64 * H, generator=_gen(L))).to(DEV)
+    sid = (torch.arange(L) * 2 // L)[None].to(DEV, torch.int32)
+    h = pkg.kernels.esmc_layer_norm(x, blk.ln1_w, blk.ln1_b, 1e-5)
+    x_mid, h2, want_x = torch.empty_like(x), torch.empty_like(h), torch.empty_like(x)
+    blk.attention(x, h, sid, 1.5, x_mid, h2)
+    want_h = pkg.kernels.esmc_layer_norm(x_mid, blk.ln1_w, blk.ln1_b, 1e-5, y_parts=blk.ffn(h2), alpha=1 / 1.5,
+                                         x_out=want_x)
+    got_x, before = torch.empty_like(x), pkg.scratch.generation(DEV)
+    blk.run(x, h, sid, 1.5, blk.ln1_w, blk.ln1_b, got_x, h)
+    assert pkg.scratch.generation(DEV) == before + 1  # one native call
+    assert torch.equal(got_x, want_x) and torch.equal(h, want_h)
+
+
+def _native_model(pkg, n=3, L=29):
+    """A model whose blocks take the native call, two sequences of it (the second of two chains), its weights."""
+    D, F_, H = 256, 320, 4
+    ps = [_weights(D, F_, seed=30 + i) for i in range(n)]
+    g = _gen(31)
+    embed, norm_w = torch.randn(33, D, generator=g), 1 + 0.1 * torch.randn(D, generator=g)
+    ids, sid = torch.randint(0, 33, (2, L), generator=g), torch.zeros(2, L, dtype=torch.int64)
+    sid[1, 15:] = 1
+    model = pkg.esmc.HipEsmc(embed, [_module_block(pkg, p, H) for p in ps], norm_w, n_heads=H)
+    return model, ids, sid, ps, embed, norm_w, H
+
+
+def test_hip_esmc_on_native_blocks(gpu_lib, pkg):
+    # the model's loop over one-call blocks: the oracle's hidden states, and the bits of the separate calls
+    n = 3
+    model, ids, sid, ps, embed, norm_w, H = _native_model(pkg, n)
+    before = pkg.scratch.generation(DEV)
+    hs = model(input_ids=ids.to(DEV), sequence_id=sid.to(DEV)).hidden_states
+    assert pkg.scratch.generation(DEV) == before + n  # one native call per block
+    x = embed.double()[ids]
+    for i, p in enumerate(ps):
+        assert float((hs[i].double().cpu() - x).abs().max()) <= 1e-2 * float(x.pow(2).mean().sqrt()) + 1e-6
+        x = oe.block_forward(p, x, sid, n_heads=H, res_scale=math.sqrt(n / 36), weights="f16")
+    last = F.layer_norm(x, (x.shape[-1],), norm_w.double(), None, 1e-5)
+    assert float((hs[n].double().cpu() - last).abs().max()) <= 1e-2 * float(last.pow(2).mean().sqrt())
+    for blk in model.layers:
+        blk.ffn = lambda h2, b=blk: pkg.esmc.EsmcBlock.ffn(b, h2)  # (a part replaced: the separate calls run)
+    before = pkg.scratch.generation(DEV)
+    assert torch.equal(model(input_ids=ids.to(DEV), sequence_id=sid.to(DEV)).hidden_states, hs)
+    assert pkg.scratch.generation(DEV) > before + n
+
+
+def test_hip_esmc_native_graph_replay(gpu_lib, pkg):
+    # the model on native blocks captured as one HIP graph, its rows in the shared scratch: every replay has the
+    # bits of the eager call, with other eager calls between the replays
+    model, ids, sid, *_ = _native_model(pkg)
+    ids, sid = ids.to(DEV), sid.to(DEV)
+    ref = model(input_ids=ids, sequence_id=sid).hidden_states.clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        hs = model(input_ids=ids, sequence_id=sid).hidden_states
+    held = pkg.scratch.current(DEV)
+    for i in range(3):
+        hs.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(hs, ref), i
+        assert not torch.equal(model(input_ids=(ids + i + 1) % 33, sequence_id=sid).hidden_states, ref)
+        torch.cuda.synchronize()
+    assert pkg.scratch.current(DEV) is held
+
+
 def _native_block(pkg, seed=0):
     """A small block that takes the native call, its input, and its output from there."""
     D, F_, H, L = 256, 320, 4, 33
