@@ -112,7 +112,7 @@ double q8_plan_cost(const Q8Plan& p, int M, int K, int N) {
 // up to two workgroups per CU where K is split, so that the partials stay within 80 MiB on 256 CUs. It is taken
 // where its estimate is lower and the scratch at hand holds its partials, and only where those are no fewer bytes
 // than the 64-row form's, so that no call is taken with less scratch than that form needs. Measured at M = 512,
-// 700, 900 and 1100, 64-row form / this, us: 2560 -> 10240 45 / 50, 64 / 51, 87 / 51, 103 / 96 (78 with the row
+// 700, 900 and 1100, 64-row form / this, us: 2560 -> 10240 45 / 50, 64 / 51, 87 / 51, 104 / 104 (75 with the row
 // split below); 2560 -> 7680 35 / 46, 51 / 47, 63 / 49, 80 / 50; 5120 -> 2560 26 / 33, 31 / 38, 37 / 42, 60 / 47;
 // 2560 -> 2560 21 / 30, 19 / 32, 22 / 36, 35 / 37; 10240 -> 2560 42 / 44, 59 / 56, 71 / 66, 112 / 76.
 constexpr double kQ8BigGroupUs = 1.1, kQ8BigFixedUs = 5.5, kQ8FixedUs = 6.0;
@@ -135,8 +135,8 @@ Q8Plan q8_plan_big(int M, int K, int N, double* cost) {
     }
   }
   // Where the tiles leave a last round mostly empty: whole rounds of them, then the remaining rows on 64-row
-  // tiles in a launch of their own, if the estimate is lower (2560 -> 10240 at M = 1100 107 -> 78 us, at
-  // 2200 154 -> 135; 2560 -> 7680 at M = 1300 91 -> 76, at 1500 110 -> 78).
+  // tiles in a launch of their own, if the estimate is lower (2560 -> 10240 at M = 1100 104 -> 75 us, at
+  // 2200 154 -> 133; 2560 -> 7680 at M = 1300 88 -> 72, at 1500 107 -> 77).
   const long long rows = tiles / cus * cus / p.ntiles * esm::kQ8BigM;
   if (rows > 0 && rows < M) {
     Q8Plan rest = q8_plan_nb(M - (int)rows, K, N, p.nb);
@@ -390,6 +390,8 @@ static bool stream_project(int C, int B, int L) {
 // launches in the workspace planes a | b | x | n (x / 256 as in the narrow path):
 //   n = LN_in(z) (cell-major)  ->  a, b = gate(n W^T) (channel-major, GATE_CM)  ->  x = a b^T
 //   ->  y = LN_mix(x) (cell-major, into plane a)  ->  out = [z +] (y W_e^T) * sigmoid(n W_g^T)
+// At C = 256 one launch takes the place of the first two (stream_project; plane n is then not used) and one of
+// the last two (stream_emit): three to five launches.
 static int tmu_forward_wide(const esm_half* z, const esm_half* mask, const float* ln_in_w, const float* ln_in_b,
                             float ln_in_eps, const esm_half* w_bundle, const float* ln_mix_w, const float* ln_mix_b,
                             float ln_mix_eps, const esm_half* w_emit, const esm_half* w_gate, esm_half* out,
@@ -782,8 +784,9 @@ static bool narrow_transition(int C, int H, bool swiglu) {
 
 // At C = 256 the whole transition is one cell-stationary kernel when its tiles of 256 cells reach more
 // than a quarter of the CUs. Below that the split into three launches, which spreads a small grid over
-// more CUs, is shorter (us, three launches against one, SwiGLU H = 1024 on 256 CUs: L = 76 53 / 70, L =
-// 100 60 / 72, L = 128 (64 tiles) 68 / 75, L = 160 120 / 79, L = 238 174 / 108; ReLU L = 128 59 / 54). At
+// more CUs, is shorter (us, three launches against one, H = 1024 on 256 CUs, SwiGLU: L = 76 53 / 69, L = 100
+// 58 / 69, L = 128 (64 tiles) 64 / 70, L = 129 105 / 70, L = 160 115 / 73, L = 238 171 / 100; ReLU: L = 76
+// 44 / 49, L = 100 52 / 49, L = 128 56 / 50, L = 129 91 / 51: the line is where both forms gain). At
 // C = 128 the register-resident kernel is the shorter one at most sizes (L = 238 26 / 24, L = 476 81 / 98).
 static bool stream_transition(int C, int H, size_t ncells) {
   return C == 256 && (size_t)H * C <= (1u << 29) && 4 * ((ncells + 255) / 256) > (size_t)cu_count();

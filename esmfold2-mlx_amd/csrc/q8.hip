@@ -429,9 +429,9 @@ __global__ __launch_bounds__(NWQ * 64, 1) void q8_linear_kernel(Q8Args p) {
 // dequantised once, a share per wave, into LDS (fp16, the same values), and every wave multiplies its 64 x 80
 // outputs (4 x 5 of v_mfma_f32_16x16x32_f16) from there. x comes by loads that write LDS, a ring of three
 // groups; the codes of a 128-k step wait in registers, two steps ahead. One barrier per group. A group takes
-// ~1.1 us (2,300 cycles against 1,280 of MFMAs on a SIMD): the dequantisation and the requests of all waves
-// precede their products. M = 1100: 2560 -> 7680 80 -> 50 us (0.86 PFLOP/s), 5120 -> 2560 60 -> 47, 10240 -> 2560
-// 112 -> 76; M = 1024: 2560 -> 10240 103 -> 59.
+// ~1.2 us, of it 1,280 cycles of MFMAs on a SIMD (the matrix cores are busy in 32-36% of a launch's cycles): the
+// dequantisation and the requests of all waves precede their products. M = 1100: 2560 -> 7680 82 -> 53 us (0.82
+// PFLOP/s), 5120 -> 2560 61 -> 48, 10240 -> 2560 113 -> 76; M = 1024: 2560 -> 10240 88 -> 57.
 namespace {
 constexpr int BGM = kQ8BigM, BGN = 32 * kQ8TileNbWide, BGT = 512;
 constexpr int BXS = BGM * 128, BWS = BGN * 128;      // bytes of a group of x and of dequantised weights

@@ -101,10 +101,11 @@ DEV void cs_lds_fence() {  // a wave's own LDS operations complete in order: a c
 // LN(z) stays in 64 registers as the B operand of the first GEMM, its 32 hidden units per step
 // become the B operand of the second one where they stand, and the output's 128 accumulators
 // start as z. The weights (96 KB per 64 units) come from L2 once per 256 cells.
-// Bound by the matrix cores' power: the loop runs them at ~72% of its cycles, and under that load
-// the shader clock falls to ~1.6 GHz (2.2 without the MFMAs). L=238, C=256, H=1024: SwiGLU 174 ->
-// 108 us, ReLU 133 -> 77; L=476: 656 -> 406 and 513 -> 288 (89 GFLOP at L=238: 0.83 PFLOP/s). What is
-// not the loop (~20 us at one tile per CU): z's arrival, the LayerNorm, the stores.
+// Bound by the matrix cores' load: over a launch at L=476 they are busy in 44% of the cycles (32% at L=238, 222
+// tiles on 256 CUs), at a clock below 1.8 GHz (2.2 in the contraction). C=256, H=1024, back to back: L=238
+// SwiGLU 171 -> 100 us, ReLU 129 -> 69; L=476 655 -> 377 and 496 -> 261 (89 GFLOP at L=238: 0.89 PFLOP/s); a
+// call among others 173 -> 92 at L=238, SwiGLU. What is not the loop (~20 us at one tile per CU): z's arrival,
+// the LayerNorm, the stores.
 template <int C, bool SWIGLU>
 struct CsTransGeo {
   static constexpr int G = SWIGLU ? 2 : 1;             // matrices of the first GEMM
@@ -320,7 +321,7 @@ __global__ __launch_bounds__(kCsThreads, 1) void transition_stream_kernel(Transi
 }
 
 // ---- projection: a, b = (LN(z) Ws^T) * sigmoid(LN(z) Wg^T) [* mask], in FragLayout ---------------------
-// One launch in place of the LayerNorm pass and the weight-stationary GEMM. No single limit: at L=476 its 160
+// One launch in place of the LayerNorm pass and the weight-stationary GEMM. No single limit: at L=476 its 165
 // us hold ~62 us of vector work (the gates' exp and rcp above all), ~26 us of MFMAs and 68 us of memory
 // traffic, and leaving any one of them out saved 20 to 60 us, so what it loses is overlap. Tried on top and not
 // faster: the gate of a block between the products of the next one (100 us for the update at L=238 either

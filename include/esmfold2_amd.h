@@ -284,7 +284,8 @@ int q8_linear(const esm_half* x, const uint8_t* q, const esm_half* s, const esm_
  *       kernel on the same stream (deterministic). q8_linear_workspace_bytes(M, K, N)
  *       bytes, 256-byte aligned, no initialisation needed; NULL runs unsplit. A workspace
  *       that holds only the partials of the 64-row tiles (none where those need none) gets
- *       the 64-row tiles. Calls that share a workspace must not overlap in time.
+ *       the 64-row tiles. The two forms add K up in different orders, and one call may divide its
+ *       rows between them: the last bit of a row can depend on M and on its place. Calls that share a workspace must not overlap in time.
  * s and b are required either way. Same semantics and result as q8_linear
  * (mx.quantized_matmul, mlx_esmc.py:78-81); packed or not, the bits are identical.
  */
@@ -411,7 +412,8 @@ int esmc_attention(const esm_half* q, const esm_half* k, const esm_half* v, cons
 int esmc_swiglu(const esm_half* x12, esm_half* y, int M, int F, void* stream);
 
 /*
- * One whole ESMC block (mlx_esmc.py:84-102) as its nine launches on the stream, from the block's LayerNormed
+ * One whole ESMC block (mlx_esmc.py:84-102) as its eight launches on the stream (one more for each of wqkv, w1
+ * whose K is split, and for each linear whose rows are divided between tile forms), from the block's LayerNormed
  * input: x' = x + alpha * wo(attention(wqkv(h))), then x_out = x' + alpha * w2(swiglu(w1(LN2(x')))), then the
  * LayerNorm that follows (the next block's input norm, or the final one): h_out fp16 or h_out_fp32, exactly
  * one of them. The same bits as the separate calls (q8_linear_packed_ws, esmc_qk_rope, esmc_attention,
