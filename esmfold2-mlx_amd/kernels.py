@@ -7,7 +7,6 @@ torch, passes raw pointers plus the current HIP stream, and raises
 
 from __future__ import annotations
 
-import contextlib
 import ctypes
 
 import torch
@@ -15,7 +14,6 @@ import torch
 from . import capi, scratch
 
 F16 = torch.float16
-_UNGUARDED = contextlib.nullcontext()  # for a call that does not touch the shared scratch
 
 
 def _dev(t: torch.Tensor, name: str, dtype=None) -> torch.Tensor:
@@ -120,7 +118,7 @@ def transition(z, ln_w, ln_b, eps, w1, w3, w2=None, out=None):
         raise capi.EsmError(-2, f"transition: w1 {tuple(w1.shape)}, w3 {tuple(w3.shape)} for C={C}")
     out = torch.empty_like(z) if out is None else _out(out, "out", F16, z.numel())
     need = int(lib.pair_transition_workspace_bytes(B, L, C, H, int(w2 is not None)))
-    with scratch.guard(z.device) if need else _UNGUARDED:
+    with scratch.guard(z.device, need):
         ws = scratch.get(need, z.device) if need else None  # the wide path's LN(z) and hidden planes
         capi.check(lib.pair_transition_ws(z.data_ptr(), out.data_ptr(), _dev(ln_w, "ln_w", torch.float32).data_ptr(),
                                           _dev(ln_b, "ln_b", torch.float32).data_ptr(), float(eps), w1.data_ptr(),
@@ -152,7 +150,7 @@ def esmc_layer_norm(x, w, b, eps, y=None, alpha: float = 1.0, x_out=None, out=No
     hp, h32 = (None, out.data_ptr()) if fp32_out else (out.data_ptr(), None)
     if y_parts is not None:
         gen = getattr(y_parts, "generation", None)  # partials living in the shared scratch: not overwritten since
-        with _UNGUARDED if gen is None else scratch.guard(y_parts[0].device):
+        with scratch.guard(y_parts[0].device, gen is not None):
             if gen is not None:
                 scratch.check_generation(gen, y_parts[0].device, "esmc_layer_norm: y_parts")
             capi.check(lib.esmc_layer_norm_parts(x.data_ptr(), y_parts[0].data_ptr(), int(y_parts[1]), float(alpha),
@@ -474,7 +472,7 @@ def q8_linear_packed(x, codes, packed, N: int, group: int = 64):
     sb = _weight(packed, "packed", torch.int32, int(lib.q8_packed_scales_bytes(N, K)))
     y = torch.empty(M, N, dtype=F16, device=x.device)
     need = int(lib.q8_linear_workspace_bytes(M, K, N))
-    with scratch.guard(x.device) if need else _UNGUARDED:
+    with scratch.guard(x.device, need):
         ws, wp, stream = scratch.take(need, x.device) if need else (None, None, capi.stream_ptr())
         capi.check(lib.q8_linear_packed_ws(x.data_ptr(), qp, sb, y.data_ptr(), M, K, N, group, wp, need, stream))
     return y

@@ -61,7 +61,7 @@ class Q8Linear(nn.Module):
         x2 = x.reshape(-1, self.in_features).to(torch.float16).contiguous()
         M = x2.shape[0]
         n = kernels.q8_workspace_bytes(M, self.in_features, self.out_features)
-        with scratch.guard(x2.device):
+        with scratch.guard(x2.device, n):
             ws = scratch.get(n, x2.device) if n else None
             y = kernels.q8_linear_swiglu(x2, self.codes_packed, self.packed, self.out_features, GROUP, workspace=ws)
         return y.reshape(*lead, self.out_features // 2)
@@ -99,7 +99,7 @@ class Q8Linear(nn.Module):
         x2 = x.reshape(-1, self.in_features).to(torch.float16).contiguous()
         M = x2.shape[0]
         n = kernels.q8_workspace_bytes(M, self.in_features, self.out_features)
-        with scratch.guard(x2.device):
+        with scratch.guard(x2.device, n):
             ws = scratch.get(n, x2.device) if n else None  # split-K partials, only while this call runs
             y = kernels.q8_linear(x2, self.q, self.scales, self.biases, GROUP, workspace=ws, packed=sb, codes=qp)
         y = y.reshape(*lead, self.out_features)

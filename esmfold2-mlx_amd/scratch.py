@@ -26,6 +26,7 @@ Rules:
 
 from __future__ import annotations
 
+import contextlib
 import threading
 from dataclasses import dataclass
 
@@ -44,6 +45,7 @@ class _Slot:
 
 _slots: dict[int, _Slot] = {}
 _guards: dict[int, threading.RLock] = {}
+_UNGUARDED = contextlib.nullcontext()
 
 
 def _index(device) -> int:
@@ -54,8 +56,11 @@ def _index(device) -> int:
     return torch.cuda.current_device() if d.index is None else d.index
 
 
-def guard(device=None) -> threading.RLock:
-    """The lock that a user of the device's scratch holds from its ``get`` until its launches are queued."""
+def guard(device=None, nbytes: int = 1):
+    """The lock that a user of the device's scratch holds from its ``get`` until its launches are queued (for a
+    call that turns out to need none, ``nbytes`` 0, one that nobody waits for)."""
+    if not nbytes:
+        return _UNGUARDED
     idx = _index(device)
     g = _guards.get(idx)
     return _guards.setdefault(idx, threading.RLock()) if g is None else g

@@ -66,3 +66,17 @@ def test_undersized_outputs_are_refused(gpu_lib, pkg):
     pair = T.TriMulPair(T.TriMul.from_weights(p), T.TriMul.from_weights(pi))
     _refused(pkg, lambda: pair(z, out=torch.empty(1, L, L - 1, C, dtype=F16, device=DEV)))
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("dtype,lead", [(torch.float32, (4,)), (F16, (4,)), (F16, (1, 4))])
+def test_host_tensors_are_refused_by_the_linear(gpu_lib, pkg, dtype, lead):
+    # a row count that needs no scratch: the refusal is the argument check's, whichever way the call takes
+    g = torch.Generator().manual_seed(1)
+    q = torch.randint(0, 256, (320, 128), generator=g, dtype=torch.uint8)
+    s = torch.ones(320, 2, dtype=F16)
+    lin, gated = pkg.q8.Q8Linear(q, s, s), pkg.q8.Q8Linear(q, s, s).swiglu_pairs()
+    assert pkg.kernels.q8_workspace_bytes(4, 128, 320) == 0
+    for call in (lin, gated, gated.swiglu):
+        with pytest.raises(pkg.capi.EsmError) as e:
+            call(torch.zeros(*lead, 128, dtype=dtype))
+        assert e.value.code == -5, str(e.value)
